@@ -281,3 +281,20 @@ def test_read_probe_reads_every_word_once(hip, n_bytes, n_wg):
         hip.read_probe(src, n_bytes, part, n_wg + 1)           # partials too small
     hip.free(src)
     hip.free(part)
+
+
+@pytest.mark.parametrize("n", [8192, 8193, 8195, 10240, 32001, 128256, 1 << 20])
+def test_argmax_many_workgroups(hip, n):
+    say(f"[ops] argmax n={n}")
+    v = synth.gauss(35, n)
+    hv, out = hip.allocate(4 * n), hip.allocate(4)
+    last = v.copy()
+    last[-1] = last[1] = 9.0            # equal maxima: the last one
+    inf = v.copy()
+    inf[n // 2] = inf[n - 2] = np.inf   # equal infinities: the first one
+    for a in (v, last, inf, np.full(n, -np.inf, np.float32), np.full(n, -1.0, np.float32), v):
+        hip.copy_to_device(a, hv)
+        hip.argmax(hv, n, out)
+        assert int(hip.download(out, 1, np.uint32)[0]) == oracle.argmax(a)
+    hip.free(hv)
+    hip.free(out)

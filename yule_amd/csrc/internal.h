@@ -42,6 +42,9 @@ struct yule_hip_backend {
     std::mutex scratch_mu;
     void *scratch = nullptr;
     size_t scratch_size = 0;
+    // argmax's workgroup slots and ticket: allocated and zeroed at creation,
+    // left zeroed by every launch on the backend's one stream
+    void *argmax_ws = nullptr;
 };
 
 namespace yule {
@@ -203,7 +206,9 @@ int launch_rms_norm(hipStream_t stream, const float *x, const float *w, float *o
 // GQA decode attention of rotated q over cache rows 0..seq-1
 int launch_gqa_attn(hipStream_t stream, const float *q, const float *kc, const float *vc, float *out, uint32_t n_heads,
                     uint32_t n_kv, uint32_t hd, uint32_t seq);
-int launch_argmax(hipStream_t stream, const float *in, uint32_t n, uint32_t *out);
+// ws: argmax_ws_bytes() bytes, zeroed once and used by one stream
+size_t argmax_ws_bytes();
+int launch_argmax(hipStream_t stream, const float *in, uint32_t n, uint32_t *out, void *ws);
 // decode-runner steps driven by the device control block ctl = {pos, token, prompt_len}
 int launch_embed_step(hipStream_t stream, uint32_t dtype, const uint8_t *table, const uint32_t *ctl,
                       const uint32_t *prompt, uint32_t vocab, float *dst, uint32_t dim);

@@ -264,8 +264,78 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const float *__restrict__ 
     }
 }
 
-int launch_argmax(hipStream_t s, const float *in, uint32_t n, uint32_t *out) {
-    hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, in, n, out);
+// Long inputs (a vocabulary's logits): up to kArgmaxWgs workgroups scan float4s
+// grid-strided, each leaves its best (value, index) in its slot, and the one
+// that takes the last ticket picks among the slots and resets the ticket (the
+// hand-off without cache-wide fences of attn_chunk_kernel: device-scope
+// stores, completed before the ticket).  The comparison is the same total
+// order, so the answer does not depend on who is last.  128256 values: 47 us
+// in one workgroup (latency of 125 dependent steps), 5.2 us so; up to 8192
+// values one workgroup of eight steps is as fast as the hand-off.
+constexpr uint32_t kArgmaxWgs = 64, kArgmaxTicket = 2 * kArgmaxWgs;   // (words of the workspace)
+__global__ __launch_bounds__(256) void argmax_wide_kernel(const float *__restrict__ in, uint32_t n,
+                                                          uint32_t *__restrict__ out, uint32_t *__restrict__ ws) {
+    __shared__ float rv[4];
+    __shared__ uint32_t ri[4];
+    const uint32_t tid = threadIdx.x, nwg = gridDim.x, n4 = n / 4;
+    float bv = -INFINITY;
+    uint32_t bi = 0;
+    auto take = [&](float v, uint32_t i) {
+        if (better(v, i, bv, bi)) { bv = v; bi = i; }
+    };
+    const float4 *in4 = reinterpret_cast<const float4 *>(in);
+    for (uint32_t i = blockIdx.x * 256 + tid; i < n4; i += nwg * 512) {
+        const uint32_t j = i + nwg * 256;
+        const float4 a = in4[i], b = in4[j < n4 ? j : i];
+        take(a.x, 4 * i); take(a.y, 4 * i + 1); take(a.z, 4 * i + 2); take(a.w, 4 * i + 3);
+        const uint32_t k = j < n4 ? j : i;   // (the same float4 again leaves the best as it is)
+        take(b.x, 4 * k); take(b.y, 4 * k + 1); take(b.z, 4 * k + 2); take(b.w, 4 * k + 3);
+    }
+    if (blockIdx.x == 0 && tid < n % 4) take(in[4 * n4 + tid], 4 * n4 + tid);
+    auto wave_best = [&]() {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+            const float ov = __shfl_xor(bv, off, 64);
+            const uint32_t oi = __shfl_xor(bi, off, 64);
+            if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+        }
+    };
+    wave_best();
+    if ((tid & 63u) == 0) { rv[tid >> 6] = bv; ri[tid >> 6] = bi; }
+    __syncthreads();
+    if (tid >= 64) return;   // the first wave does the rest
+    uint32_t last = 0;
+    if (tid == 0) {
+        for (int k = 1; k < 4; k++) take(rv[k], ri[k]);
+        __hip_atomic_store(ws + 2 * blockIdx.x, __float_as_uint(bv), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(ws + 2 * blockIdx.x + 1, bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt(0);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        last = __hip_atomic_fetch_add(ws + kArgmaxTicket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nwg - 1;
+    }
+    if (!__builtin_amdgcn_readfirstlane(last)) return;
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const uint32_t s = tid < nwg ? tid : 0u;
+    bv = __uint_as_float(__hip_atomic_load(ws + 2 * s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    bi = __hip_atomic_load(ws + 2 * s + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    wave_best();
+    if (tid == 0) {
+        out[0] = bi;
+        __hip_atomic_store(ws + kArgmaxTicket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+size_t argmax_ws_bytes() { return (kArgmaxTicket + 1) * sizeof(uint32_t); }
+
+// ws: argmax_ws_bytes() bytes, zeroed once, used by one stream
+int launch_argmax(hipStream_t s, const float *in, uint32_t n, uint32_t *out, void *ws) {
+    if (n <= 8192) {
+        hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(1024), 0, s, in, n, out);
+    } else {
+        const uint32_t wgs = n / 2048 < kArgmaxWgs ? n / 2048 : kArgmaxWgs;
+        hipLaunchKernelGGL(argmax_wide_kernel, dim3(wgs), dim3(256), 0, s, in, n, out, static_cast<uint32_t *>(ws));
+    }
     return check_launch("argmax");
 }
 
@@ -623,7 +693,7 @@ int yule_hip_argmax(yule_hip_backend *be, yule_buffer in, uint32_t n, yule_buffe
     void *po;
     int rc;
     if ((rc = f32buf(be, in, n, &pi, "argmax (in)")) || (rc = get_buffer(be, out, 4, &po, "argmax (out)"))) return rc;
-    return launch_argmax(be->stream, pi, n, (uint32_t *)po);
+    return launch_argmax(be->stream, pi, n, (uint32_t *)po, be->argmax_ws);
 }
 
 }  // extern "C"

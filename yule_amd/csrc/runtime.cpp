@@ -136,6 +136,11 @@ int yule_hip_create(int device, yule_hip_backend **out) {
         delete be;
         return rc;
     }
+    if ((rc = hip_error(hipMalloc(&be->argmax_ws, argmax_ws_bytes()), "create: argmax workspace")) ||
+        (rc = hip_error(hipMemsetAsync(be->argmax_ws, 0, argmax_ws_bytes(), be->stream), "create: argmax workspace"))) {
+        yule_hip_destroy(be);
+        return rc;
+    }
     *out = be;
     return YULE_OK;
 }
@@ -147,6 +152,7 @@ int yule_hip_destroy(yule_hip_backend *be) {
     for (auto &kv : be->buffers) hipFree(kv.second.ptr);
     be->buffers.clear();
     if (be->scratch) hipFree(be->scratch);
+    if (be->argmax_ws) hipFree(be->argmax_ws);
     for (hipEvent_t e : be->timer)
         if (e) hipEventDestroy(e);
     if (be->cap_exec) hipGraphExecDestroy(be->cap_exec);
