@@ -283,6 +283,44 @@ def test_read_probe_reads_every_word_once(hip, n_bytes, n_wg):
     hip.free(part)
 
 
+# positions around the 16-position and 1024-thread steps, head sizes around the
+# 16-dim slices, offsets and strides that are and are not multiples of 4
+@pytest.mark.parametrize("hd, seq, n_kv, shift", [(64, 1, 4, 0), (64, 777, 4, 0), (128, 1024, 2, 0), (80, 257, 3, 0),
+                                                  (20, 65, 2, 0), (7, 63, 3, 0), (64, 1025, 2, 1), (66, 300, 1, 0)])
+def test_attn_score_value_shapes(hip, hd, seq, n_kv, shift):
+    say(f"[ops] attn_score / attn_value hd={hd} seq={seq} kv={n_kv} shift={shift}")
+    kvs = n_kv * hd + shift
+    q, kc, vc = synth.gauss(31, 2 * hd), synth.gauss(32, (seq, kvs)), synth.gauss(33, (seq, kvs))
+    off = (n_kv - 1) * hd + shift
+    hq, hk, hv, hs, ho = hip.upload(q), hip.upload(kc), hip.upload(vc), hip.allocate(4 * seq), hip.allocate(4 * (hd + 3))
+    hip.attn_score(hq, hk, hs, hd, seq, hd, off, kvs)
+    s = hip.download(hs, seq)
+    q64, k64, v64 = q[hd:].astype(np.float64), kc[:, off:off + hd].astype(np.float64), vc[:, off:off + hd].astype(np.float64)
+    # f32 sums of n terms: error at most n * 2^-24 of the sum of magnitudes
+    assert np.all(np.abs(s - k64 @ q64 / math.sqrt(hd)) <= (hd + 4) * 2.0 ** -24 * (np.abs(k64) @ np.abs(q64)) / math.sqrt(hd))
+    hip.softmax(hs, hs, seq)
+    p = hip.download(hs, seq)
+    e = np.exp(s.astype(np.float64) - s.max())
+    # exp of a rounded difference, relative: |difference| * 2^-24 plus expf's 2 ulp, the sum's and the product's rounding
+    assert close(p / (e / e.sum()), 1.0, (np.ptp(s) + seq / 256 + 16) * 2.0 ** -23)
+    hip.attn_value(hs, hv, ho, hd, seq, off, kvs, 3)
+    p64 = p.astype(np.float64)
+    assert np.all(np.abs(hip.download(ho, hd + 3)[3:] - p64 @ v64) <= (seq + 4) * 2.0 ** -24 * (p64 @ np.abs(v64)))
+    for b in (hq, hk, hv, hs, ho):
+        hip.free(b)
+
+
+@pytest.mark.parametrize("n", [1, 1024, 1025, 8192, 8193])
+def test_softmax_sizes(hip, n):
+    say(f"[ops] softmax n={n}")
+    x = synth.gauss(34, n, 3.0)
+    hx = hip.upload(x)
+    hip.softmax(hx, hx, n)
+    e = np.exp(x.astype(np.float64) - x.max())
+    assert close(hip.download(hx, n) / (e / e.sum()), 1.0, (np.ptp(x) + n / 256 + 16) * 2.0 ** -23)
+    hip.free(hx)
+
+
 @pytest.mark.parametrize("n", [8192, 8193, 8195, 10240, 32001, 128256, 1 << 20])
 def test_argmax_many_workgroups(hip, n):
     say(f"[ops] argmax n={n}")
