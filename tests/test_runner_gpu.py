@@ -510,3 +510,27 @@ def test_runner_long_context_split(hip):
             logits = ref.forward(want[-1])
     assert list(toks) == want
     run.close()
+
+
+@pytest.mark.parametrize("hd,heads,kv,pieces", [(32, 8, 8, (1, 15, 17)), (64, 12, 4, (33, 1, 14)), (128, 4, 2, (16, 47)),
+                                                (256, 2, 1, (20, 13)), (64, 8, 1, (7, 290)), (64, 16, 2, (530,))])
+def test_runner_prefill_attention_tiles(hip, hd, heads, kv, pieces):
+    """Batched prefill in pieces: query tiles of 16 rows whole and ragged, both
+    workgroup widths, one to eight heads per KV head, every head size: logits
+    after each piece vs the float64 forward (two layers, so that every row of
+    the first feeds the result)."""
+    from yule_amd.model import LlamaConfig
+    cfg = LlamaConfig(n_layers=2, dim=hd * heads, n_heads=heads, n_kv_heads=kv, ff_dim=512, vocab=256, max_seq=544)
+    m = SyntheticModel.generate(cfg, seed=40 + hd, scheme="Q4_K")
+    say(f"[runner] prefill attention hd {hd} heads {heads}/{kv} pieces {pieces}")
+    toks = synth.uniform_tokens(41, sum(pieces), cfg.vocab)
+    run, f64, at = HipRunner(hip, m), NpForward(m), 0
+    try:
+        for n in pieces:
+            got = run.prefill_batched(toks[at:at + n])
+            for t in toks[at:at + n]:
+                want = f64.forward(int(t))
+            at += n
+            assert np.max(np.abs(got - want)) <= tolerance_bar(want), f"after {at} tokens"
+    finally:
+        run.close()
