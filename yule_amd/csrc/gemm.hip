@@ -1287,12 +1287,14 @@ namespace {
 // that small-M launches keep all CUs busy without a partial second round.
 // Tile width along the weight rows: 256 (eight waves) halves the X bytes
 // each weight tile is multiplied against and measured 5-30% faster once M
-// fills the CUs with wide tiles (M >= 1024; Q6_K, whose dequant is dearer,
-// from M >= 512); 128 (four waves) below that.  YULE_GEMM_BN overrides.
-uint32_t gemm_bn(uint32_t m, uint32_t dtype) {
+// fills the CUs with wide tiles (M >= 1024; Q6_K, whose dequant is dearer
+// and whose 128-row kernels run one wave per SIMD either way, from 512, and
+// with bf16 X above 128: 4096 x 14336 at M = 129 94.7 -> 78.5 us, 333 161 -> 119, 4096 x
+// 4096 at M = 400 63 -> 57); 128 (four waves) below that.  YULE_GEMM_BN overrides.
+uint32_t gemm_bn(uint32_t m, uint32_t dtype, bool f32x) {
     static const int env = env_int("YULE_GEMM_BN", 0);
     if (env == 128 || env == 256) return (uint32_t)env;
-    return m >= 1024 || (dtype == YULE_DTYPE_Q6_K && m >= 512) ? 256u : 128u;
+    return m >= 1024 || (dtype == YULE_DTYPE_Q6_K && (m >= 512 || (!f32x && m > 128))) ? 256u : 128u;
 }
 
 // Tile height: 64 rows for M <= 64, and for f32 X up to M = 128 (its two
@@ -1457,7 +1459,7 @@ struct GemmWork {
 static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool f32x) {
     GemmWork g;
     g.q4 = dtype == YULE_DTYPE_Q4_K || dtype == YULE_DTYPE_Q5_K;   // min term: X sub-block sums
-    g.bn = gemm_bn(m, dtype);
+    g.bn = gemm_bn(m, dtype, f32x);
     g.bm = gemm_bm(m, f32x, dtype, g.bn);
     g.skinny = gemm_skinny(m, n_cols, dtype, f32x);
     g.ks = g.skinny ? gemm_skinny_splits(n_rows, n_cols) : gemm_splits(m, n_rows, n_cols, g.bn, g.bm, gemm_wgs_per_cu(dtype, g.bm, g.bn, f32x));
