@@ -267,6 +267,37 @@ def test_gemm_f32_full_range_and_repeat(hip, dt):
         assert np.max(np.abs(a[M - 1] - ref)) <= tolerance_bar(ref)
 
 
+def test_gemm_operand_tiles(hip):
+    """The operand-tile path at the edges of its tiles, all formats, bf16 and
+    f32 X (tests/gemm_tiled_check.py, in a child process because the switch
+    that sends small products there is read once per process)."""
+    import os
+    import subprocess
+    from pathlib import Path
+    say("[gemm] operand tiles")
+    r = subprocess.run([sys.executable, str(Path(__file__).with_name("gemm_tiled_check.py"))],
+                       env=dict(os.environ, YULE_GEMM_TILED_MIN="1"), capture_output=True, text=True, timeout=110)
+    out = r.stdout.strip().splitlines()
+    assert r.returncode == 0 and out and out[-1].startswith("ok"), r.stdout[-2000:] + r.stderr[-4000:]
+    say(f"[gemm] {out[-1]}")
+
+
+# products that the size rule itself sends to the operand tiles, one K split
+# and several, and the first row count on either side of the line
+@pytest.mark.parametrize("dt,M,N,K", [(DType.Q6_K, 129, 3900, 3072), (DType.Q6_K, 128, 3900, 3072),
+                                      (DType.Q8_0, 300, 5000, 2048), (DType.Q4_K, 700, 11264, 2048),
+                                      (DType.Q5_K, 699, 11264, 2048), (DType.Q4_0, 200, 4096, 4096)],
+                         ids=lambda v: getattr(v, "name", str(v)))
+def test_gemm_f32_many_rows(hip, dt, M, N, K):
+    say(f"[gemm f32] many rows {dt.name} M={M} N={N} K={K}")
+    w = synth.gen_quant(dt, 130 + M, N, K)
+    x = synth.gauss(131 + K, (M, K))
+    y = run_gemm_f32(hip, dt, w, x, M, N, K)
+    for m in (0, M // 2, M - 1):
+        ref = oracle.qmv_f64(int(dt), w, x[m], N, K)
+        assert np.max(np.abs(y[m] - ref)) <= tolerance_bar(ref), f"row {m}"
+
+
 def test_gemm_errors(hip):
     w = synth.gen_quant(DType.Q4_K, 1, 16, 256)
     hw, hx, hy = hip.upload(w), hip.allocate(2 * 256 * 4), hip.allocate(4 * 16 * 4)

@@ -45,6 +45,7 @@
 #include <type_traits>
 #include <string>
 
+#include "gemm_tiled.h"
 #include "qmv_common.h"
 
 namespace yule {
@@ -1453,10 +1454,13 @@ struct GemmWork {
     size_t part_bytes, total;
     size_t n_x, n_sub, n_y;
     uint32_t ks, bn, bm, tail;
-    bool q4, skinny;
+    bool q4, skinny, tiled;
+    TiledPlan tp;
 };
 
-static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool f32x) {
+// tiled: the product over operand tiles may serve it (their workspace is
+// larger than the static one)
+static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool f32x, bool tiled = true) {
     GemmWork g;
     g.q4 = dtype == YULE_DTYPE_Q4_K || dtype == YULE_DTYPE_Q5_K;   // min term: X sub-block sums
     g.bn = gemm_bn(m, dtype, f32x);
@@ -1467,7 +1471,15 @@ static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t
     g.n_x = (size_t)m * n_cols;
     g.n_sub = (size_t)m * (n_cols / 32);
     g.n_y = (size_t)m * n_rows;
+    g.tiled = tiled && gemm_tiled_plan(m, n_rows, n_cols, dtype, f32x, &g.tp);
+    if (g.tiled) g.ks = g.tp.ks;
     g.part_bytes = g.ks > 1 ? ((g.ks * g.n_y * sizeof(float) + 255) & ~(size_t)255) : 0;
+    if (g.tiled) {
+        auto up = [](size_t b) { return (b + 1023) & ~(size_t)1023; };   // (tiles_layout's pieces)
+        g.total = 1024 + g.part_bytes + up(g.tp.w_bytes) + up(g.tp.we_bytes) + up(g.tp.s_bytes) + up(g.tp.t_bytes) +
+                  (f32x ? 2 : 1) * up(g.tp.x_bytes) + up(g.tp.xe_bytes) + (size_t)m * sizeof(float) + 1024;
+        return g;
+    }
     g.total = g.part_bytes + ((f32x ? 2 : 1) * g.n_x + (g.q4 ? 2 * g.n_sub : 0)) * sizeof(_Float16) + 256 +
               (size_t)m * sizeof(float) + 256;
     return g;
@@ -1475,6 +1487,24 @@ static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t
 
 // Enqueue the pre-pass and the product(s) of one call into workspace ws.
 static GemmW one_matrix(const uint8_t *w, uint32_t n_rows) { return GemmW{{w, w, w}, n_rows, n_rows}; }
+
+// pending's reduction produces this X (checked before it is left to the pre-pass)
+static int check_pending(const GemmRed *pending, const void *x, bool f32x, uint32_t m, uint32_t n_cols, bool glu) {
+    if (pending && pending->ks > 1 &&
+        (!f32x || pending->y != x || pending->m != m || pending->ny != (glu ? 2 : 1) * n_cols))
+        return set_error(YULE_ERR_INVALID, "quantized_gemm: pending reduction does not produce this X");
+    return YULE_OK;
+}
+
+// A product's split-K partials into y, or left to the next product's pre-pass (defer)
+static int finish_splits(hipStream_t s, const GemmWork &g, const float *part, float *y, uint32_t m, uint32_t n_rows,
+                         bool accumulate, GemmRed *defer) {
+    if (defer) *defer = GemmRed{part, y, g.ks > 1 ? g.ks : 0u, n_rows, m, accumulate};
+    if (g.ks <= 1 || defer) return YULE_OK;
+    hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((g.n_y + 255) / 256)), dim3(256), 0, s, part, y,
+                       (uint64_t)g.n_y, g.ks, accumulate ? 1u : 0u);
+    return check_launch("quantized_gemm: split-K reduction");
+}
 
 // accumulate: Y += the product (no K-half tail then: its atomic adds would
 // add into Y in either order)
@@ -1484,14 +1514,35 @@ static int gemm_enqueue(hipStream_t s, const GemmW &w, const void *x, bool f32x,
                         GemmRed *defer = nullptr, const GemmRed *pending = nullptr) {
     uint8_t *b = static_cast<uint8_t *>(ws);
     float *part = g.ks > 1 ? reinterpret_cast<float *>(b) : nullptr;
+    int rc = check_pending(pending, x, f32x, m, n_cols, glu);
+    if (rc) return rc;
+    if (g.tiled) {
+        uint8_t *at = b + g.part_bytes;
+        auto take = [&](size_t bytes) {
+            at = reinterpret_cast<uint8_t *>((reinterpret_cast<uintptr_t>(at) + 1023) & ~(uintptr_t)1023);
+            uint8_t *p = at;
+            at += bytes;
+            return p;
+        };
+        TiledPass a{{w.w[0], w.w[1], w.w[2]}, w.s1, w.s2, m, n_rows, n_cols, dtype, f32x, accumulate, nullptr, nullptr,
+                    nullptr, take(g.tp.w_bytes), take(g.tp.we_bytes), take(g.tp.s_bytes), take(g.tp.t_bytes), nullptr,
+                    g.ks > 1 ? part : y};
+        a.xh = take(g.tp.x_bytes);
+        a.xl = f32x ? take(g.tp.x_bytes) : nullptr;
+        a.xe = take(g.tp.xe_bytes);
+        float *const rs = reinterpret_cast<float *>(take((size_t)m * sizeof(float)));
+        a.rowscale = rs;
+        rc = launch_x_tiles(s, x, f32x, m, n_cols, g.tp.ext, norm_w, eps, glu, const_cast<void *>(a.xh),
+                            const_cast<void *>(a.xl), const_cast<void *>(a.xe), rs, pending);
+        if (rc || (rc = launch_gemm_tiled(s, g.tp, a))) return rc;
+        return finish_splits(s, g, part, y, m, n_rows, accumulate, defer);
+    }
     _Float16 *xh = reinterpret_cast<_Float16 *>(b + g.part_bytes);
     _Float16 *xl = f32x ? xh + g.n_x : nullptr;
     _Float16 *xs_hi = g.q4 ? xh + (f32x ? 2 : 1) * g.n_x : nullptr, *xs_lo = g.q4 ? xs_hi + g.n_sub : nullptr;
     float *rowscale = reinterpret_cast<float *>(
         (reinterpret_cast<uintptr_t>(xh + (f32x ? 2 : 1) * g.n_x + (g.q4 ? 2 * g.n_sub : 0)) + 255) & ~(uintptr_t)255);
     const bool red = pending && pending->ks > 1;
-    if (red && (!f32x || pending->y != x || pending->m != m || pending->ny != (glu ? 2 : 1) * n_cols))
-        return set_error(YULE_ERR_INVALID, "quantized_gemm: pending reduction does not produce this X");
     if (f32x)
         hipLaunchKernelGGL(gemm_xprep_kernel<true>, dim3(m), dim3(256), 0, s, x, norm_w, n_cols, eps, glu ? 1u : 0u,
                            xh, xl, xs_hi, xs_lo, rowscale, red ? pending->part : nullptr, red ? pending->ks : 0u,
@@ -1499,19 +1550,11 @@ static int gemm_enqueue(hipStream_t s, const GemmW &w, const void *x, bool f32x,
     else
         hipLaunchKernelGGL(gemm_xprep_kernel<false>, dim3(m), dim3(256), 0, s, x, norm_w, n_cols, eps, 0u, xh, xl,
                            xs_hi, xs_lo, rowscale, nullptr, 0u, 0u, m, 0u);
-    int rc = check_launch("quantized_gemm: x pre-pass");
-    if (rc) return rc;
+    if ((rc = check_launch("quantized_gemm: x pre-pass"))) return rc;
     const GemmPass p{w, xh, xl, xs_hi, xs_lo, rowscale, g.ks > 1 ? part : y, m, n_rows, n_cols, g.ks, g.bn, g.bm,
                      accumulate ? 0u : g.tail, accumulate ? 1u : 0u};
     if ((rc = g.skinny ? launch_gemm_skinny(s, p) : launch_gemm_dt(s, dtype, p))) return rc;
-    if (defer) *defer = GemmRed{part, y, g.ks > 1 ? g.ks : 0u, n_rows, m, accumulate};
-    if (g.ks > 1 && defer) return YULE_OK;   // summed by the next product's pre-pass
-    if (g.ks > 1) {
-        hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((g.n_y + 255) / 256)), dim3(256), 0, s, part, y,
-                           (uint64_t)g.n_y, g.ks, accumulate ? 1u : 0u);
-        if ((rc = check_launch("quantized_gemm: split-K reduction"))) return rc;
-    }
-    return YULE_OK;
+    return finish_splits(s, g, part, y, m, n_rows, accumulate, defer);
 }
 
 // ---- static workspace of the allocation-free entry point
@@ -1563,7 +1606,7 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
     if (weights == y || weights == x) return set_error(YULE_ERR_INVALID, std::string(what) + ": weights alias x or y");
     if (!m || !n_rows) return YULE_OK;
     if (!n_cols) return launch_fill(be->stream, (float *)py, 0.f, (uint64_t)m * n_rows);
-    const GemmWork g = gemm_work(m, n_rows, n_cols, dtype, f32x);
+    const GemmWork g = gemm_work(m, n_rows, n_cols, dtype, f32x, !noalloc);
     if (noalloc) {
         if (g.total > kStaticWorkspaceBytes)
             return set_error(YULE_ERR_INVALID, std::string(what) + ": this call needs " + std::to_string(g.total) +
