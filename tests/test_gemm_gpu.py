@@ -282,6 +282,25 @@ def test_gemm_operand_tiles(hip):
     say(f"[gemm] {out[-1]}")
 
 
+# Q6_K: partials of the 256-wide tiles' K splits that do and do not fit the
+# static workspace (then the 128-wide tiles serve the call)
+@pytest.mark.parametrize("M", [130, 384, 511])
+def test_gemm_noalloc_q6k_partials(hip, M):
+    N = K = 4096
+    say(f"[gemm noalloc] Q6_K M={M}")
+    w = synth.gen_quant(DType.Q6_K, 140, N, K)
+    xb = bf16_bits(synth.gauss(141, (M, K)))
+    hw, hx, hy = hip.upload(w), hip.upload(xb), hip.allocate(4 * M * N)
+    hip.quantized_gemm_noalloc(hw, hx, hy, M, N, K, DType.Q6_K)
+    y = hip.download(hy, (M, N))
+    xf = bf16_to_f32(xb).reshape(M, K)
+    for m in (0, M - 1):
+        ref = oracle.qmv_f64(int(DType.Q6_K), w, xf[m], N, K)
+        assert np.max(np.abs(y[m] - ref)) <= tolerance_bar(ref), f"row {m}"
+    for h in (hw, hx, hy):
+        hip.free(h)
+
+
 # products that the size rule itself sends to the operand tiles, one K split
 # and several, and the first row count on either side of the line
 @pytest.mark.parametrize("dt,M,N,K", [(DType.Q6_K, 129, 3900, 3072), (DType.Q6_K, 128, 3900, 3072),

@@ -1459,11 +1459,13 @@ struct GemmWork {
 };
 
 // tiled: the product over operand tiles may serve it (their workspace is
-// larger than the static one)
-static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool f32x, bool tiled = true) {
+// larger than the static one); narrow: Q6_K's 128-wide tiles below 512 rows,
+// whose K splits need half the partials
+static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool f32x, bool tiled = true,
+                          bool narrow = false) {
     GemmWork g;
     g.q4 = dtype == YULE_DTYPE_Q4_K || dtype == YULE_DTYPE_Q5_K;   // min term: X sub-block sums
-    g.bn = gemm_bn(m, dtype, f32x);
+    g.bn = gemm_bn(m, dtype, f32x || narrow);
     g.bm = gemm_bm(m, f32x, dtype, g.bn);
     g.skinny = gemm_skinny(m, n_cols, dtype, f32x);
     g.ks = g.skinny ? gemm_skinny_splits(n_rows, n_cols) : gemm_splits(m, n_rows, n_cols, g.bn, g.bm, gemm_wgs_per_cu(dtype, g.bm, g.bn, f32x));
@@ -1606,8 +1608,9 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
     if (weights == y || weights == x) return set_error(YULE_ERR_INVALID, std::string(what) + ": weights alias x or y");
     if (!m || !n_rows) return YULE_OK;
     if (!n_cols) return launch_fill(be->stream, (float *)py, 0.f, (uint64_t)m * n_rows);
-    const GemmWork g = gemm_work(m, n_rows, n_cols, dtype, f32x, !noalloc);
+    GemmWork g = gemm_work(m, n_rows, n_cols, dtype, f32x, !noalloc);
     if (noalloc) {
+        if (g.total > kStaticWorkspaceBytes) g = gemm_work(m, n_rows, n_cols, dtype, f32x, false, true);
         if (g.total > kStaticWorkspaceBytes)
             return set_error(YULE_ERR_INVALID, std::string(what) + ": this call needs " + std::to_string(g.total) +
                                                    " bytes of workspace, above the static " +
