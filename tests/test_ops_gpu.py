@@ -191,6 +191,15 @@ def test_gqa_decode_attn_long(hip, hd, nh, nkv, seq):
     run_gqa_case(hip, hd, nh, nkv, seq)
 
 
+@pytest.mark.parametrize("hd,nh,nkv,seq", [(64, 8, 8, 20481), (128, 8, 8, 12097), (128, 16, 2, 82001),
+                                          (64, 48, 16, 7937), (128, 32, 32, 2033)])
+def test_gqa_decode_attn_chunk_lengths(hip, hd, nh, nkv, seq):
+    """Split-KV chunks of 320, 192, 320, 256 and 128 positions with a short
+    last chunk (one key, or part of a 16-key sub-tile)."""
+    say(f"[ops] gqa_decode_attn chunks hd={hd} heads={nh}/{nkv} seq={seq}")
+    run_gqa_case(hip, hd, nh, nkv, seq)
+
+
 def test_gqa_decode_attn_limits(hip):
     """More than 8 query heads per KV head: the per-head kernel up to 16384
     positions, refused above; above 262144 positions refused for any shape."""

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <string>
 
+#include "attn_tile.h"
 #include "blocks.h"
 #include "internal.h"
 #include "qmv_common.h"
@@ -1098,7 +1099,7 @@ __global__ __launch_bounds__(NT) void attn_step_kernel(const float *__restrict__
 // the chunk maximum m_c, the sum l_c = sum_t exp(s_t - m_c) and the
 // unnormalised output o_c = sum_t exp(s_t - m_c) V_t; phase 2 combines the
 // chunks: out = sum_c exp(m_c - M) o_c / sum_c exp(m_c - M) l_c.
-// The chunk length is a function of the sequence length alone (split_chunk),
+// The chunk length is a function of the sequence length and KV heads alone,
 // evaluated on the device in decode steps, so a captured graph sized for
 // max_seq serves every position; workgroups past the last chunk exit.
 constexpr uint32_t kSplitMaxGroup = 8;      // query heads per KV head
@@ -1111,6 +1112,22 @@ __host__ __device__ inline uint32_t split_chunk(uint32_t seq, uint32_t n_kv) {
     const uint32_t target = 512;
     if (n_kv * ((seq + 255) / 256) >= target) return 256;
     if (n_kv * ((seq + 127) / 128) >= target) return 128;
+    return 64;
+}
+
+// The same for attn_split_tile_kernel.  Below 16 KV heads the chunks are 192
+// and 320 long: workgroups in flight start a chunk of rows apart, and with
+// 4096-byte rows (8 heads of 128) a power of two puts them on the same memory
+// channels.  32/8 heads x 128, 15001 positions: 192 22.1 us, 128 28.4, 256
+// 28.8; 60000 positions: 320 81.8, 256 91.2, 128 101.9 (and the combine 5.8
+// against 10.1).  A position of 16 or more heads covers the channels by
+// itself, and 128 fills the chip earlier (32 heads x 128, 2000 positions: 128
+// 11.8 us, 192 15.0).
+__host__ __device__ inline uint32_t split_tile_chunk(uint32_t seq, uint32_t n_kv) {
+    if (n_kv >= 16) return split_chunk(seq, n_kv);
+    const uint32_t target = 512;
+    if (n_kv * ((seq + 319) / 320) >= target) return 320;
+    if (n_kv * ((seq + 191) / 192) >= target) return 192;
     return 64;
 }
 
@@ -1254,7 +1271,148 @@ __global__ __launch_bounds__(256) void attn_split_kernel(const float *__restrict
     if (tid < G) ml[(size_t)(h0 + tid) * max_chunks + chunk] = make_float2(m[tid], l[tid]);
 }
 
-// Phase 2: one workgroup per query head.
+// Phase 1 on the f32 matrix instructions (head sizes 64 and 128): the same
+// partials and step handling, with the group's query heads as the columns of
+// an attention tile (attn_tile.h; columns past G repeat the last head).  A
+// workgroup's four waves take the chunk's sub-tiles of 16 keys in turn,
+// operands straight from the cache, the next K loaded under the softmax and
+// the next V under the next scores: a wave has 16 rows in flight, read in
+// 64-byte (K) and 256-byte (V) pieces, where the kernel above reads a K row
+// with one to four lanes.  Bound by memory.  Against that kernel (us, with the
+// combine): 32/8 heads x 128: 1024 positions 11.4 -> 9.1, 15001 35.4 -> 27.1,
+// 60000 304 -> 88; 32/4 x 64, 15001: 35.3 -> 13.2; 32/32 x 128, 15001: 289 ->
+// 91 (6.0 TB/s).  The chunk maxima are in the tile's base-2 units.
+template <uint32_t HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void attn_split_tile_kernel(
+    const float *__restrict__ q, const float *__restrict__ k, const float *__restrict__ v, float *__restrict__ kc,
+    float *__restrict__ vc, const float *__restrict__ cos_t, const float *__restrict__ sin_t,
+    const uint32_t *__restrict__ ctl, float *__restrict__ part, float2 *__restrict__ ml, uint32_t G, uint32_t n_kv,
+    uint32_t seq_host, uint32_t max_chunks) {
+    using T = AttnTile<HD>;
+    constexpr uint32_t OS = HD + 4, half = HD / 2;
+    __shared__ __align__(16) float os[4 * kSplitMaxGroup * OS];
+    __shared__ float ms[4][kSplitMaxGroup], ls[4][kSplitMaxGroup];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), kvh = blockIdx.x, chunk = blockIdx.y;
+    const bool step = ctl != nullptr;
+    const uint32_t seq = step ? ctl[0] + 1 : seq_host, pos = seq - 1;
+    const uint32_t C = split_tile_chunk(seq, n_kv), c0 = chunk * C;
+    if (c0 >= seq) return;   // uniform over the workgroup
+    const uint32_t end = c0 + C < seq ? c0 + C : seq, h0 = kvh * G;
+    T st;
+    st.init(q + (size_t)(h0 + (c < G ? c : G - 1u)) * HD, g);
+    // four dims (two rotation pairs) at 16 s + 4 g of a row, rotated by position pos
+    auto rotate = [&](float4 x, uint32_t s) {
+        const size_t j = (size_t)pos * half + 8 * s + 2 * g;
+        const float2 cs = *reinterpret_cast<const float2 *>(cos_t + j), sn = *reinterpret_cast<const float2 *>(sin_t + j);
+        return make_float4(x.x * cs.x - x.y * sn.x, x.x * sn.x + x.y * cs.x, x.z * cs.y - x.w * sn.y,
+                           x.z * sn.y + x.w * cs.y);
+    };
+    if (step) {
+#pragma unroll
+        for (uint32_t s = 0; s < T::NS; s++) st.q[s] = rotate(st.q[s], s);
+    }
+    const uint32_t kvs = n_kv * HD;
+    float *kb = kc + (size_t)kvh * HD, *vb = vc + (size_t)kvh * HD;
+    float4 kr[T::NS];
+    float vr[4][T::NG][T::VW];
+    // (a sub-tile's base is uniform; lane offsets of at most 15 rows fit 32 bits:
+    // above that the two caches would exceed the card)
+    auto load_k = [&](uint32_t k0) {
+        const char *base = reinterpret_cast<const char *>(kb + (size_t)k0 * kvs);
+        const uint32_t off = 4 * (min(c, pos - k0) * kvs + 4 * g);
+#pragma unroll
+        for (uint32_t s = 0; s < T::NS; s++) kr[s] = *reinterpret_cast<const float4 *>(base + off + 64 * s);
+    };
+    auto load_v = [&](uint32_t k0) {
+        const char *base = reinterpret_cast<const char *>(vb + (size_t)k0 * kvs);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+            const uint32_t off = 4 * (min(4 * g + r, pos - k0) * kvs + 4 * c);
+#pragma unroll
+            for (uint32_t i = 0; i < T::NG; i++) {
+                const float4 x = *reinterpret_cast<const float4 *>(base + off + 256 * i);
+                vr[r][i][0] = x.x; vr[r][i][1] = x.y; vr[r][i][2] = x.z; vr[r][i][3] = x.w;
+            }
+        }
+    };
+    uint32_t k0 = c0 + 16 * wave;
+    if (k0 < end) {
+        load_k(k0);
+        load_v(k0);
+    }
+    for (; k0 < end; k0 += 64) {
+        const bool tail = k0 + 16 > seq, own = step && pos - k0 < 16u;
+        if (own && k0 + c == pos) {   // the new row: from the launch before, and into the cache
+#pragma unroll
+            for (uint32_t s = 0; s < T::NS; s++) {
+                kr[s] = rotate(*reinterpret_cast<const float4 *>(k + (size_t)kvh * HD + 16 * s + 4 * g), s);
+                *reinterpret_cast<float4 *>(kb + (size_t)pos * kvs + 16 * s + 4 * g) = kr[s];
+            }
+        }
+        if (own || tail) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) {
+                const uint32_t t = k0 + 4 * g + r;
+#pragma unroll
+                for (uint32_t i = 0; i < T::NG; i++) {
+                    if (own && t == pos) {
+                        const float4 x = *reinterpret_cast<const float4 *>(v + (size_t)kvh * HD + 64 * i + 4 * c);
+                        vr[r][i][0] = x.x; vr[r][i][1] = x.y; vr[r][i][2] = x.z; vr[r][i][3] = x.w;
+                        *reinterpret_cast<float4 *>(vb + (size_t)pos * kvs + 64 * i + 4 * c) = x;
+                    } else if (t >= seq) {   // (weight 0: the value must be finite)
+                        vr[r][i][0] = vr[r][i][1] = vr[r][i][2] = vr[r][i][3] = 0.f;
+                    }
+                }
+            }
+        }
+        f4v sc[2] = {f4v{0, 0, 0, 0}, f4v{0, 0, 0, 0}};
+#pragma unroll
+        for (uint32_t s = 0; s < T::NS; s++) st.score(sc[s & 1u], kr[s], s);
+        const bool more = k0 + 64 < end;
+        if (more) load_k(k0 + 64);
+        sc[0] += sc[1];
+        st.softmax(sc[0], k0, g, pos, tail);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++)
+#pragma unroll
+            for (uint32_t i = 0; i < T::NG; i++) st.value(sc[0][r], vr[r][i], i);
+        if (more) load_v(k0 + 64);
+    }
+    float l = st.l;
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (c < G) {
+        st.store(os + (wave * kSplitMaxGroup + c) * OS, g);
+        if (g == 0) {
+            ms[wave][c] = st.m;
+            ls[wave][c] = l;
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < G * (HD / 4); i += 256) {
+        const uint32_t h = i / (HD / 4), d = 4 * (i % (HD / 4));
+        const float M = fmaxf(fmaxf(ms[0][h], ms[1][h]), fmaxf(ms[2][h], ms[3][h]));
+        float L = 0.f;
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (uint32_t w = 0; w < 4; w++) {
+            const float f = __builtin_amdgcn_exp2f(ms[w][h] - M);
+            const float4 o = *reinterpret_cast<const float4 *>(os + (w * kSplitMaxGroup + h) * OS + d);
+            L += f * ls[w][h];
+            a.x += f * o.x; a.y += f * o.y; a.z += f * o.z; a.w += f * o.w;
+        }
+        const size_t at = (size_t)(h0 + h) * max_chunks + chunk;
+        *reinterpret_cast<float4 *>(part + at * HD + d) = a;
+        if (d == 0) ml[at] = make_float2(M, L);
+    }
+}
+
+// Phase 2: one workgroup per query head; lanes own four dims and a residue
+// class of the chunks (four in flight), summed through LDS.  118 chunks of 32
+// heads x 128: 10.8 us with one thread per dim walking the chunks, 4.9 us so.
+// BASE2: the maxima are of base-2 exponents (attn_split_tile_kernel).
+template <bool BASE2>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restrict__ part,
                                                            const float2 *__restrict__ ml,
                                                            const uint32_t *__restrict__ ctl, float *__restrict__ out,
@@ -1262,9 +1420,10 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restri
                                                            uint32_t max_chunks) {
     __shared__ float wt[kSplitMaxChunks];
     __shared__ float red[16];
+    __shared__ float4 os[256];
     const uint32_t h = blockIdx.x, tid = threadIdx.x;
     const uint32_t seq = ctl ? ctl[0] + 1 : seq_host;
-    const uint32_t C = split_chunk(seq, n_kv), n_ch = (seq + C - 1) / C;
+    const uint32_t C = BASE2 ? split_tile_chunk(seq, n_kv) : split_chunk(seq, n_kv), n_ch = (seq + C - 1) / C;
     const float2 *mh = ml + (size_t)h * max_chunks;
     float mx = -INFINITY;
     for (uint32_t c = tid; c < n_ch; c += 256) mx = fmaxf(mx, mh[c].x);
@@ -1272,22 +1431,41 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restri
     float lsum = 0.f;
     for (uint32_t c = tid; c < n_ch; c += 256) {
         const float2 v = mh[c];
-        const float e = expf(v.x - mx);
+        const float e = BASE2 ? __builtin_amdgcn_exp2f(v.x - mx) : expf(v.x - mx);
         wt[c] = e;
         lsum += e * v.y;
     }
     lsum = block_sum(lsum, red);   // its barriers also publish wt[]
     const float inv = 1.0f / lsum;
-    const float *ph = part + (size_t)h * max_chunks * hd;
-    for (uint32_t d = tid; d < hd; d += 256) {
-        float a0 = 0.f, a1 = 0.f;
-        uint32_t c = 0;
-        for (; c + 1 < n_ch; c += 2) {
-            a0 += wt[c] * ph[(size_t)c * hd + d];
-            a1 += wt[c + 1] * ph[(size_t)(c + 1) * hd + d];
+    const uint32_t nd4 = hd / 4, ng = 256 / nd4, d4 = tid % nd4, gi = tid / nd4;
+    const float4 *ph = reinterpret_cast<const float4 *>(part + (size_t)h * max_chunks * hd) + d4;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (gi < ng) {
+        uint32_t c = gi;
+        for (; c + 3 * ng < n_ch; c += 4 * ng) {
+            float4 p[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) p[u] = ph[(size_t)(c + u * ng) * nd4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                const float w = wt[c + u * ng];
+                a.x += w * p[u].x; a.y += w * p[u].y; a.z += w * p[u].z; a.w += w * p[u].w;
+            }
         }
-        if (c < n_ch) a0 += wt[c] * ph[(size_t)c * hd + d];
-        out[(size_t)h * hd + d] = (a0 + a1) * inv;
+        for (; c < n_ch; c += ng) {
+            const float4 p = ph[(size_t)c * nd4];
+            const float w = wt[c];
+            a.x += w * p.x; a.y += w * p.y; a.z += w * p.z; a.w += w * p.w;
+        }
+    }
+    os[tid] = a;
+    __syncthreads();
+    if (tid < nd4) {
+        for (uint32_t j = 1; j < ng; j++) {
+            const float4 p = os[j * nd4 + tid];
+            a.x += p.x; a.y += p.y; a.z += p.z; a.w += p.w;
+        }
+        reinterpret_cast<float4 *>(out + (size_t)h * hd)[tid] = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
     }
 }
 
@@ -1562,22 +1740,36 @@ int launch_attn_split(hipStream_t s, const float *q, const float *k, const float
     float *part = static_cast<float *>(scratch);
     float2 *ml = reinterpret_cast<float2 *>(part + (size_t)n_heads * mc * hd);
     const uint32_t seq_host = ctl ? 0u : seq_cap;
-    const dim3 grid(n_kv, ctl ? mc : (seq_cap + split_chunk(seq_cap, n_kv) - 1) / split_chunk(seq_cap, n_kv));
+    const bool tile = hd == 64 || hd == 128;
+    const uint32_t C = tile ? split_tile_chunk(seq_cap, n_kv) : split_chunk(seq_cap, n_kv);
+        const dim3 grid(n_kv, ctl ? mc : (seq_cap + C - 1) / C);
+#define YULE_SPLIT_ARGS q, k, v, kc, vc, cos_t, sin_t, ctl, part, ml
 #define YULE_SPLIT_CASE(G)                                                                                       \
     case G:                                                                                                      \
-        hipLaunchKernelGGL(attn_split_kernel<G>, grid, dim3(256), 0, s, q, k, v, kc, vc, cos_t, sin_t, ctl, part, \
-                           ml, n_kv, hd, seq_host, mc);                                                          \
+        hipLaunchKernelGGL(attn_split_kernel<G>, grid, dim3(256), 0, s, YULE_SPLIT_ARGS, n_kv, hd, seq_host, mc); \
         break;
-    switch (n_heads / n_kv) {
-        YULE_SPLIT_CASE(1) YULE_SPLIT_CASE(2) YULE_SPLIT_CASE(3) YULE_SPLIT_CASE(4)
-        YULE_SPLIT_CASE(5) YULE_SPLIT_CASE(6) YULE_SPLIT_CASE(7) YULE_SPLIT_CASE(8)
-    default: return set_error(YULE_ERR_UNSUPPORTED, "split attention: more than 8 query heads per KV head");
-    }
+    const uint32_t group = n_heads / n_kv;
+    if (!group || group > kSplitMaxGroup)
+        return set_error(YULE_ERR_UNSUPPORTED, "split attention: more than 8 query heads per KV head");
+    if (hd == 64)
+        hipLaunchKernelGGL(attn_split_tile_kernel<64>, grid, dim3(256), 0, s, YULE_SPLIT_ARGS, group, n_kv, seq_host, mc);
+    else if (hd == 128)
+        hipLaunchKernelGGL(attn_split_tile_kernel<128>, grid, dim3(256), 0, s, YULE_SPLIT_ARGS, group, n_kv, seq_host, mc);
+    else
+        switch (group) {
+            YULE_SPLIT_CASE(1) YULE_SPLIT_CASE(2) YULE_SPLIT_CASE(3) YULE_SPLIT_CASE(4)
+            YULE_SPLIT_CASE(5) YULE_SPLIT_CASE(6) YULE_SPLIT_CASE(7) YULE_SPLIT_CASE(8)
+        }
 #undef YULE_SPLIT_CASE
+#undef YULE_SPLIT_ARGS
     int rc = check_launch("attn_split");
     if (rc) return rc;
-    hipLaunchKernelGGL(attn_combine_kernel, dim3(n_heads), dim3(256), 0, s, part, ml, ctl, out, n_kv, hd, seq_host,
-                       mc);
+    if (tile)
+        hipLaunchKernelGGL(attn_combine_kernel<true>, dim3(n_heads), dim3(256), 0, s, part, ml, ctl, out, n_kv, hd,
+                           seq_host, mc);
+    else
+        hipLaunchKernelGGL(attn_combine_kernel<false>, dim3(n_heads), dim3(256), 0, s, part, ml, ctl, out, n_kv, hd,
+                           seq_host, mc);
     return check_launch("attn_combine");
 }
 
