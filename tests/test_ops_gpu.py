@@ -170,6 +170,16 @@ def run_gqa_case(hip, hd, nh, nkv, seq, tol=1e-5):
     assert err <= tol, f"max error {err:.3g}"
 
 
+@pytest.mark.parametrize("hd,nh,nkv,seq", [(hd, nh, nkv, seq) for hd, nh, nkv in ((64, 4, 4), (128, 20, 2))
+                                          for seq in (1, 16, 17, 128, 257, 511, 512)])
+def test_gqa_decode_attn_per_head(hip, hd, nh, nkv, seq):
+    """The one-workgroup-per-head kernel at the ends of a wave's positions and
+    of its rounds; more than 8 heads per KV head, which never run split-KV,
+    stay on it at 512."""
+    say(f"[ops] per-head gqa_decode_attn hd={hd} heads={nh}/{nkv} seq={seq}")
+    run_gqa_case(hip, hd, nh, nkv, seq)
+
+
 @pytest.mark.parametrize("hd,nh,nkv,seq", [(64, 8, 2, 1), (64, 8, 2, 65), (64, 32, 4, 384), (128, 32, 8, 1000),
                                           (80, 8, 2, 77), (32, 4, 4, 33), (64, 24, 8, 300), (64, 40, 8, 500),
                                           (256, 16, 2, 129), (128, 56, 8, 257), (64, 4, 4, 700)])

@@ -152,6 +152,34 @@ def test_runner_hd64_attention_paths(hip, chunks, split_min, monkeypatch):
     assert [int(t) for t in out] == want
 
 
+@pytest.mark.parametrize("hd,chunks,split_min", [(64, "1", None), (64, "0", None), (128, "0", None), (64, "1", "600")])
+def test_runner_attention_rounds(hip, hd, chunks, split_min, monkeypatch):
+    """Decode steps around the positions where the one-workgroup-per-head
+    kernel's waves and rounds end (16 or 8 positions a wave, 256 or 128 a
+    round) up to the split-KV threshold, with q rotated by the Q/K/V launch
+    or in the attention launch; and the chunked kernel, which serves launches
+    of more than 512 rows.  The rows between come from the batched prompt
+    pass; logits vs the oracle."""
+    from yule_amd.model import LlamaConfig
+    monkeypatch.setenv("YULE_ATTN_CHUNKS", chunks)
+    if split_min:
+        monkeypatch.setenv("YULE_ATTN_SPLIT_MIN", split_min)
+    m = SyntheticModel.generate(LlamaConfig(n_layers=2, dim=512, n_heads=512 // hd, n_kv_heads=2, ff_dim=512,
+                                            vocab=512, max_seq=640), seed=23)
+    say(f"[runner] attention rounds hd {hd}, chunks {chunks}, split from {split_min}")
+    run, ref = HipRunner(hip, m), oracle.Runner(m, n_threads=4)
+    toks, pos = synth.uniform_tokens(33, 520, m.cfg.vocab), 0
+    for stop in (14, 126, 254, 506):
+        run.prefill_batched(toks[pos:stop])
+        for t in toks[pos:stop]:
+            ref.forward(int(t))
+        for i in range(stop, stop + 5):
+            got, want = run.decode_step(int(toks[i])), ref.forward(int(toks[i]))
+            assert np.max(np.abs(got - want)) <= tolerance_bar(want), f"position {i}"
+        pos = stop + 5
+    run.close()
+
+
 @pytest.mark.parametrize("scheme,dim,hd", [("Q4_K", 512, 64), ("Q6_K", 1024, 64), ("Q8_0", 512, 128),
                                             ("Q6_K", 512, 128), ("Q4_K", 2048, 128)])
 def test_runner_attention_formats_and_head_sizes(hip, scheme, dim, hd):

@@ -148,7 +148,8 @@ int launch_embed_rows(hipStream_t stream, uint32_t dtype, const uint8_t *table, 
 int gemm_static_workspace_init(int device);
 // decode-step attention over a cache that already holds row ctl[0] and a
 // rotated q (after a kEpiRope Q/K/V launch): one workgroup per (query head,
-// chunk), chunks combined in-launch; hd 64 or 128 (attn_chunk_len != 0)
+// chunk), chunks combined in-launch, or one per head for few rows of hd 64;
+// hd 64 or 128 (attn_chunk_len != 0)
 uint32_t attn_chunk_len(uint32_t hd);
 size_t attn_chunk_scratch_bytes(uint32_t n_heads, uint32_t hd, uint32_t max_rows);
 int launch_attn_chunks(hipStream_t stream, const float *q, const float *kc, const float *vc, const uint32_t *ctl,

@@ -51,8 +51,8 @@ struct yule_hip_runner {
     uint32_t split_min = 0;
     void *attn_ws = nullptr;
     // shorter steps, when the Q/K/V launch can rotate and write the cache
-    // itself (kEpiRope): chunked attention with in-launch combine (partials
-    // and per-head tickets in chunk_ws, zeroed at creation)
+    // itself (kEpiRope): launch_attn_chunks, whose chunked kernel keeps its
+    // partials and per-head tickets in chunk_ws, zeroed at creation
     void *chunk_ws = nullptr;
     // batched prefill (prefill_rows): row buffers for max_seq rows and the
     // GEMM workspace, allocated at the first batched prefill
@@ -579,7 +579,7 @@ int yule_hip_runner_create(yule_hip_backend *be, const yule_model_desc *d, yule_
     if ((rc = dev_alloc(r, kArgmaxSlots * sizeof(unsigned long long), reinterpret_cast<void **>(&r->amax))))
         return fail(rc);
     // chunked attention for steps below the split threshold (YULE_ATTN_CHUNKS=0
-    // at creation: the one-workgroup-per-head kernel instead)
+    // at creation: q rotated in the attention launch, one workgroup per head)
     const char *ce = getenv("YULE_ATTN_CHUNKS");
     if ((!ce || atoi(ce) != 0) && attn_chunk_len(hd) &&
         (rc = dev_alloc(r, attn_chunk_scratch_bytes(r->n_heads, hd, std::min(r->max_seq, r->split_min)), &r->chunk_ws)))
