@@ -104,6 +104,30 @@ def test_gemm_wide_tiles(hip, dt, M, N, K):
         hip.free(h)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 256), (13, 77, 2304), (16, 200, 4096), (5, 33, 8448), (16, 4096, 4096),
+                                   (17, 200, 4096)])
+def test_gemm_few_rows_q8_0(hip, M, N, K):
+    """Q8_0, M <= 16 on weights of up to 2^24 elements: the one-launch kernel
+    (one unit for one wave, nine and 33 units over 16 waves, a ragged last
+    tile), bf16 and f32 X, every row vs the oracle; f32 X spread over 60 powers
+    of two and a row near the top of the range, whose outputs are finite;
+    M = 17 is the tile kernel's again."""
+    dt = DType.Q8_0
+    say(f"[gemm] few rows Q8_0 M={M} N={N} K={K}")
+    w = synth.gen_quant(dt, 130 + M, N, K)
+    xb = bf16_bits(synth.gauss(131 + K, (M, K)))
+    y = run_gemm(hip, dt, w, xb, M, N, K)
+    xf = bf16_to_f32(xb).reshape(M, K)
+    x32 = synth.gauss(132 + K, (M, K)) * np.exp2(np.arange(M, dtype=np.float32) * 4 - 30)[:, None].astype(np.float32)
+    if M == 13:
+        x32[12] *= np.float32(2.0 ** 102)   # quants times it pass the f32 range, the scaled outputs do not
+    y32 = run_gemm_f32(hip, dt, w, x32, M, N, K)
+    for m in range(M):
+        for got, x in ((y, xf), (y32, x32)):
+            ref = oracle.qmv_f64(int(dt), w, x[m], N, K)
+            assert np.max(np.abs(ref)) < 3e38 and np.max(np.abs(got[m] - ref)) <= tolerance_bar(ref), f"row {m}"
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 77, 1024), (5, 300, 3072), (16, 64, 2048), (17, 129, 1024),
                                    (32, 200, 3072), (32, 1000, 2048), (8, 4096, 5120), (3, 2000, 14336),
                                    (33, 1000, 2048)])

@@ -1589,6 +1589,114 @@ static void *static_workspace(int device) {
     return g_static_ptr[device];
 }
 
+// Q8_0 products of at most 16 X rows in one launch and without workspace: a
+// workgroup of 16 waves owns 16 weight rows and splits K, each wave taking
+// units of 8 blocks; per block of 32 one 16x16x32 bf16 MFMA per part of X
+// (rows = X rows, columns = weight rows, so a lane's block scale is its own
+// row's), scaled into f32 accumulators that meet in LDS.  Quants are exact in
+// bf16 and f32 X is the exact sum of three bf16 parts, so only the f32 sums
+// round.  Bound by the address work of its 8-byte weight reads and of X, which
+// every workgroup reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
+// reduction -> this): 256x1024 15.6 -> 4.6, 1030x2048 17.0 -> 8.9, 4096x4096
+// 26.4 -> 17.1 (bf16 X 20.6 -> 13.8; one row of f32 X 25.2 -> 13.3).  Larger
+// weights stay on the tiles, which read them in whole lines: 16 rows, 14336 x
+// 4096 f32 X 49.0 there and 53.1 here, bf16 X 30.1 and 45.2.
+typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
+typedef float few_f4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t kFewRows = 16;
+constexpr uint64_t kFewWeights = 1ull << 24;   // n_rows * n_cols
+
+template <bool F32>
+__global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__restrict__ w, const void *__restrict__ xv,
+                                                            float *__restrict__ y, uint32_t m, uint32_t n_rows,
+                                                            uint32_t n_cols) {
+    constexpr uint32_t NW = 16, U = 8;
+    constexpr float kDown = 0x1p-12f;   // quants reach 2^7 and a block sums 2^5: its sum stays within the largest |x|
+    __shared__ __align__(16) float red[NW][256];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), n0 = blockIdx.x * 16;
+    const uint32_t mr = c < m ? c : m - 1;
+    const uint8_t *wr = w + (size_t)(n0 + c < n_rows ? n0 + c : n_rows - 1) * (n_cols / 32) * 34;
+    const float *xf = static_cast<const float *>(xv) + (size_t)mr * n_cols + 8 * g;
+    const uint16_t *xh = static_cast<const uint16_t *>(xv) + (size_t)mr * n_cols + 8 * g;
+    few_f4 acc = {0, 0, 0, 0};
+    for (uint32_t u = wave; u < n_cols / 256; u += NW) {
+        uint2 qs[U];
+        uint16_t ds[U];
+        float4 xr[F32 ? 2 * U : U];
+#pragma unroll
+        for (uint32_t b = 0; b < U; b++) {
+            const uint8_t *blk = wr + (size_t)(u * U + b) * 34;
+            __builtin_memcpy(&ds[b], blk, 2);
+            __builtin_memcpy(&qs[b], blk + 2 + 8 * g, 8);   // 2-byte aligned
+            if constexpr (F32) {
+                const float4 *p = reinterpret_cast<const float4 *>(xf + u * 256 + b * 32);
+                xr[2 * b] = p[0];
+                xr[2 * b + 1] = p[1];
+            } else {
+                xr[b] = *reinterpret_cast<const float4 *>(xh + u * 256 + b * 32);
+            }
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < U; b++) {
+            // X as bf16 parts (one, or three that sum to the f32 exactly)
+            constexpr uint32_t NP = F32 ? 3 : 1;
+            bf8v a[NP];
+            if constexpr (F32) {
+                float x[8] = {xr[2 * b].x,     xr[2 * b].y,     xr[2 * b].z,     xr[2 * b].w,
+                              xr[2 * b + 1].x, xr[2 * b + 1].y, xr[2 * b + 1].z, xr[2 * b + 1].w};
+#pragma unroll
+                for (uint32_t part = 0; part < NP; part++) {
+                    uint32_t h[4];
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++)
+                        h[i] = __builtin_amdgcn_perm(__float_as_uint(x[2 * i + 1]), __float_as_uint(x[2 * i]),
+                                                     0x07060302u);
+                    __builtin_memcpy(&a[part], h, 16);
+#pragma unroll
+                    for (uint32_t i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
+                }
+            } else {
+                __builtin_memcpy(&a[0], &xr[b], 16);
+            }
+            uint32_t wq[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; i++) {   // two quants a dword, the upper halves of their floats
+                const uint32_t v = (i < 2 ? qs[b].x : qs[b].y) >> (16 * (i & 1u));
+                wq[i] = __builtin_amdgcn_perm(__float_as_uint((float)(int8_t)(v >> 8) * kDown),
+                                              __float_as_uint((float)(int8_t)v * kDown), 0x07060302u);
+            }
+            bf8v bw;
+            __builtin_memcpy(&bw, wq, 16);
+            few_f4 t = {0, 0, 0, 0};
+#pragma unroll
+            for (uint32_t part = 0; part < NP; part++)
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[part], bw, t, 0, 0, 0);
+            _Float16 d;
+            __builtin_memcpy(&d, &ds[b], 2);
+            const float df = (float)d;
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) acc[r] += df * t[r];
+        }
+    }
+    *reinterpret_cast<few_f4 *>(&red[wave][4 * lane]) = acc;
+    __syncthreads();
+    const uint32_t on = tid & 15u, om = tid >> 4, row = n0 + on;   // weight row and X row of a thread
+    if (om >= m || row >= n_rows) return;                          // m is at most 16
+    float sum = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < NW; i++) sum += red[i][4 * ((om >> 2) * 16 + on) + (om & 3u)];
+    y[(size_t)om * n_rows + row] = sum * (1.0f / kDown);
+}
+
+static int launch_gemm_few_q80(hipStream_t s, const uint8_t *w, const void *x, bool f32x, float *y, uint32_t m,
+                               uint32_t n_rows, uint32_t n_cols) {
+    const dim3 grid((n_rows + 15) / 16);
+    if (f32x) hipLaunchKernelGGL(gemm_few_q80_kernel<true>, grid, dim3(1024), 0, s, w, x, y, m, n_rows, n_cols);
+    else hipLaunchKernelGGL(gemm_few_q80_kernel<false>, grid, dim3(1024), 0, s, w, x, y, m, n_rows, n_cols);
+    return check_launch("quantized_gemm (few X rows)");
+}
+
 static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, bool f32x, yule_buffer y, uint32_t m,
                       uint32_t n_rows, uint32_t n_cols, uint32_t dtype, const char *what, bool noalloc = false) {
     if (!be) return set_error(YULE_ERR_INVALID, "null backend");
@@ -1608,6 +1716,7 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
     if (weights == y || weights == x) return set_error(YULE_ERR_INVALID, std::string(what) + ": weights alias x or y");
     if (!m || !n_rows) return YULE_OK;
     if (!n_cols) return launch_fill(be->stream, (float *)py, 0.f, (uint64_t)m * n_rows);
+    const bool few = dtype == YULE_DTYPE_Q8_0 && m <= kFewRows && (uint64_t)n_rows * n_cols <= kFewWeights;
     GemmWork g = gemm_work(m, n_rows, n_cols, dtype, f32x, !noalloc);
     if (noalloc) {
         if (g.total > kStaticWorkspaceBytes) g = gemm_work(m, n_rows, n_cols, dtype, f32x, false, true);
@@ -1617,9 +1726,11 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
                                                    std::to_string(kStaticWorkspaceBytes) + "-byte one");
         void *ws = static_workspace(be->device);
         if (!ws) return set_error(YULE_ERR_HIP, std::string(what) + ": static workspace not set up for this device");
+        if (few) return launch_gemm_few_q80(be->stream, (const uint8_t *)pw, px, f32x, (float *)py, m, n_rows, n_cols);
         return gemm_enqueue(be->stream, one_matrix((const uint8_t *)pw, n_rows), px, f32x, (float *)py, m, n_rows,
                             n_cols, dtype, g, ws);
     }
+    if (few) return launch_gemm_few_q80(be->stream, (const uint8_t *)pw, px, f32x, (float *)py, m, n_rows, n_cols);
     ScratchLease lease;   // held until every launch below is enqueued
     if ((rc = get_scratch(be, g.total, &lease))) return rc;
     return gemm_enqueue(be->stream, one_matrix((const uint8_t *)pw, n_rows), px, f32x, (float *)py, m, n_rows, n_cols,
