@@ -25,6 +25,21 @@ __host__ __device__ inline uint32_t gemm_ext_cols(uint32_t dtype, uint32_t k) {
     return dtype == YULE_DTYPE_Q4_K || dtype == YULE_DTYPE_Q5_K ? (3 * (k / 32) + 31) / 32 * 32 : 0;
 }
 
+// Scales: gemm_tiled_kernel copies a stage's (32 k) rows of the scale array
+// [k / gran][np] beside its tiles.  The row a walk over the stages starts
+// from at stage `stage`, and by how many rows it moves on when it comes to the
+// next one, `stage`: the extra range (from stage main_s on) has no scales of
+// its own, and its copies (in the wait counts, never read) stay on the last
+// row of the main range.
+__host__ __device__ constexpr uint32_t tile_scale_rows(uint32_t gran) { return gran == 16 ? 2u : 1u; }   // per stage
+__host__ __device__ inline uint32_t tile_scale_row(uint32_t gran, uint32_t stage, uint32_t main_s) {
+    const uint32_t s = stage < main_s ? stage : main_s - 1u;
+    return gran == 16 ? 2 * s : gran == 32 ? s : s >> 3;
+}
+__host__ __device__ inline uint32_t tile_scale_step(uint32_t gran, uint32_t stage, uint32_t main_s) {
+    return stage >= main_s || (gran == 256 && (stage & 7u)) ? 0u : tile_scale_rows(gran);
+}
+
 struct TiledPlan {
     uint32_t gran;                // k per weight scale (256, 32 or 16)
     uint32_t ks, n_chunk;         // K splits; weight rows per pass (all of them with splits)

@@ -373,7 +373,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     constexpr uint32_t BM = kTiledBm, BN = kTiledBn, NBUF = SW == 1 ? 3 : 2;
     constexpr uint32_t MT = BM / 64, NT = BN / 64;                 // MFMA tiles per wave
     constexpr uint32_t AB = BM / 32 * 2, BBK = BN / 32 * 2;        // 1 KB blocks per stage: one X operand, the weights
-    constexpr uint32_t SCW = GRAN == 16 ? 2 : 1;                  // scale rows per stage, 1 KB (256 floats) each
+    constexpr uint32_t SCW = tile_scale_rows(GRAN);               // 1 KB (256 floats) each
     constexpr uint32_t NB = SW * AB + BBK;
     constexpr uint32_t BUF = (NB + SCW) * 1024;
     __shared__ __align__(1024) uint8_t lds[NBUF * BUF];
@@ -425,8 +425,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const uint32_t blk = 4 * i + wave, idx = blk < SW * AB ? blk % AB : blk - SW * AB;
             off[i] = ((idx >> 1) * row_blocks + (idx & 1u)) * 1024 + lane * 16;
         }
-        const uint32_t sm = main ? fs : main_s - 1u, srow = GRAN == 16 ? 2 * sm : GRAN == 32 ? sm : sm >> 3;
-        ps = reinterpret_cast<const uint8_t *>(scale + (size_t)srow * np + tn * BN + 64 * wave);
+        ps = reinterpret_cast<const uint8_t *>(scale + (size_t)tile_scale_row(GRAN, fs, main_s) * np + tn * BN + 64 * wave);
     };
     auto fetch = [&](uint32_t b) {   // stage fs into buffer b, then on to the next (the last one again past the end)
         const uint32_t dst = lds0 + b * BUF;
@@ -445,7 +444,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             pa += 2048;
             pl += 2048;
             pb += 2048;
-            if (GRAN != 256 || (fs & 7u) == 0) ps += (size_t)SCW * np * 4;
+            ps += (size_t)tile_scale_step(GRAN, fs, main_s) * np * 4;
             if (fs == main_s) point();
         }
     };
