@@ -1,6 +1,9 @@
-"""The operand-tile GEMM's plan on the CPU: what the kernel addresses lies
-inside the workspace that the plan sizes.  A small host program includes the
-kernel's own addressing (gemm_tiled.h) and asks the built library for plans."""
+"""The GEMM kernels' host-checkable rules on the CPU.  The operand-tile plan:
+what the kernel addresses lies inside the workspace that the plan sizes (a
+small host program includes the kernel's own addressing, gemm_tiled.h, and
+asks the built library for plans).  The copies into LDS that are issued as
+inline assembly: a wait state between the write of M0 and the load."""
+import re
 import shutil
 import subprocess
 from pathlib import Path
@@ -65,3 +68,16 @@ def host_run(tmp_path_factory):
 def test_scale_rows_stay_inside_the_scales(host_run):
     r = host_run("scales", SCALE_WALK, YULE_GEMM_TILED_MIN="1")
     assert r.returncode == 0 and r.stdout.count(".") >= 35, r.stdout + r.stderr
+
+
+def test_wait_state_between_m0_and_lds_loads():
+    """gfx9: one wait state between a scalar write of M0 and a load into LDS;
+    the compiler adds it for its own loads and does not look into asm text."""
+    found = 0
+    for src in sorted([*CSRC.glob("*.hip"), *CSRC.glob("*.h")]):
+        for text in re.findall(r'asm volatile\(\s*((?:"(?:[^"\\]|\\.)*"\s*)+)', src.read_text()):
+            ops = [o.split()[0:2] for o in re.sub(r'"\s*"', "", text).strip().strip('"').replace("\\t", "").split("\\n")]
+            for a, b in zip(ops, ops[1:]):
+                assert not (a[1:2] == ["m0,"] and "lds" in b[0]), f"{src.name}: {text}"
+            found += any("lds" in o[0] for o in ops)
+    assert found >= 3

@@ -750,6 +750,8 @@ __global__ __launch_bounds__(2 * BN) __attribute__((amdgpu_waves_per_eu(gemm_wav
     // are in flight, i.e. stricter; none falls after a stage's copy, since
     // the stage's weight registers were already covered by the previous
     // stage's explicit wait, which the compiler does account for.
+    // The wait state that a load into LDS needs after a scalar write of M0 is
+    // explicit for the same reason.
     // Scheduling barriers keep the copies first in their stage, ahead of the
     // weight loads whose count the waits rely on.
     typedef __attribute__((address_space(3))) _Float16 *lds_h;
@@ -764,7 +766,7 @@ __global__ __launch_bounds__(2 * BN) __attribute__((amdgpu_waves_per_eu(gemm_wav
             const _Float16 *src = xcur + (size_t)m * K + k0 + 8u * c;
             const uint32_t dst = __builtin_amdgcn_readfirstlane(
                 (uint32_t)reinterpret_cast<uintptr_t>((lds_h)(xbuf(b) + (64u * wave + NTH * i) * 8u)));
-            asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "m0");
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(dst) : "m0");
         }
         __builtin_amdgcn_sched_barrier(0);
     };

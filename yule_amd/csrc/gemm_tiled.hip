@@ -402,12 +402,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((lds_b)lds);
     // 64 x W dwords from base + off into LDS; outside the compiler's memory
     // model (its loads and waits know nothing of it): every wait for it is
-    // explicit
+    // explicit, and so is the wait state that a load into LDS needs after a
+    // scalar write of M0 (the compiler does not look for hazards in here)
     auto copy = [&](auto w, const uint8_t *base, uint32_t off, uint32_t dst) {
         if constexpr (decltype(w)::value == 4)
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "m0");
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "m0");
         else
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(dst) : "m0");
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(dst) : "m0");
     };
     // where the next stage's copies come from: this wave's blocks i of the
     // tiles (their offsets fixed but for the step to the extra k range)
