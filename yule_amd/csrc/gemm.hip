@@ -1734,7 +1734,13 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
     }
     if (few) return launch_gemm_few_q80(be->stream, (const uint8_t *)pw, px, f32x, (float *)py, m, n_rows, n_cols);
     ScratchLease lease;   // held until every launch below is enqueued
-    if ((rc = get_scratch(be, g.total, &lease))) return rc;
+    if ((rc = get_scratch(be, g.total, &lease))) {
+        // no room on the card, or a capture, under which the workspace cannot
+        // grow: the plan that needs least
+        const GemmWork least = gemm_work(m, n_rows, n_cols, dtype, f32x, false, true);
+        if (least.total >= g.total || get_scratch(be, least.total, &lease)) return rc;
+        g = least;
+    }
     return gemm_enqueue(be->stream, one_matrix((const uint8_t *)pw, n_rows), px, f32x, (float *)py, m, n_rows, n_cols,
                         dtype, g, lease.ptr);
 }
@@ -1743,19 +1749,26 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
 // runner's batched prefill)
 bool yule::gemm_supports(uint32_t dtype, uint32_t n_cols) { return gemm_dtype_ok(dtype) && n_cols % 256 == 0; }
 
-size_t yule::gemm_f32_workspace_bytes(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype) {
-    return gemm_work(m, n_rows, n_cols, dtype, true).total;
+static GemmWork f32_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, size_t ws_bytes) {
+    const GemmWork g = gemm_work(m, n_rows, n_cols, dtype, true);
+    return g.total <= ws_bytes ? g : gemm_work(m, n_rows, n_cols, dtype, true, false);
+}
+
+size_t yule::gemm_f32_workspace_bytes(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool least) {
+    return gemm_work(m, n_rows, n_cols, dtype, true, !least).total;
 }
 
 int yule::launch_gemm_f32(hipStream_t s, const uint8_t *w, const float *x, float *y, uint32_t m, uint32_t n_rows,
-                          uint32_t n_cols, uint32_t dtype, void *ws, bool accumulate, const float *norm_w, float eps,
-                          bool glu, GemmRed *defer, const GemmRed *pending) {
+                          uint32_t n_cols, uint32_t dtype, void *ws, size_t ws_bytes, bool accumulate,
+                          const float *norm_w, float eps, bool glu, GemmRed *defer, const GemmRed *pending) {
     if (!gemm_dtype_ok(dtype) || n_cols % 256) return set_error(YULE_ERR_UNSUPPORTED, "gemm: format or shape");
     if (glu && norm_w) return set_error(YULE_ERR_INVALID, "gemm: SwiGLU input and RMSNorm together");
     if (defer) defer->ks = 0;
     if (!m || !n_rows) return YULE_OK;
-    return gemm_enqueue(s, one_matrix(w, n_rows), x, true, y, m, n_rows, n_cols, dtype,
-                        gemm_work(m, n_rows, n_cols, dtype, true), ws, accumulate, norm_w, eps, glu, defer, pending);
+    const GemmWork g = f32_work(m, n_rows, n_cols, dtype, ws_bytes);
+    if (g.total > ws_bytes) return set_error(YULE_ERR_INVALID, "gemm: workspace too small");
+    return gemm_enqueue(s, one_matrix(w, n_rows), x, true, y, m, n_rows, n_cols, dtype, g, ws, accumulate, norm_w, eps,
+                        glu, defer, pending);
 }
 
 // Several matrices of one format and width that share X, as one product
@@ -1770,15 +1783,15 @@ bool yule::gemm_multi_ok(uint32_t dtype, uint32_t n_cols, const uint32_t *rows, 
 }
 
 size_t yule::gemm_f32_multi_workspace_bytes(uint32_t m, const uint32_t *rows, uint32_t n_mat, uint32_t n_cols,
-                                            uint32_t dtype) {
+                                            uint32_t dtype, bool least) {
     uint32_t total = 0;
     for (uint32_t i = 0; i < n_mat; i++) total += rows[i];
-    return gemm_work(m, total, n_cols, dtype, true).total;
+    return gemm_f32_workspace_bytes(m, total, n_cols, dtype, least);
 }
 
 int yule::launch_gemm_f32_multi(hipStream_t s, const uint8_t *const *w, const uint32_t *rows, uint32_t n_mat,
                                 const float *x, float *y, uint32_t m, uint32_t n_cols, uint32_t dtype, void *ws,
-                                const float *norm_w, float eps, GemmRed *defer, const GemmRed *pending) {
+                                size_t ws_bytes, const float *norm_w, float eps, GemmRed *defer, const GemmRed *pending) {
     if (!gemm_multi_ok(dtype, n_cols, rows, n_mat)) return set_error(YULE_ERR_UNSUPPORTED, "gemm: format or shape");
     if (defer) defer->ks = 0;
     if (!m) return YULE_OK;
@@ -1786,8 +1799,9 @@ int yule::launch_gemm_f32_multi(hipStream_t s, const uint8_t *const *w, const ui
     const uint32_t total = rows[0] + (n_mat > 1 ? rows[1] : 0) + (n_mat > 2 ? rows[2] : 0);
     g.s1 = n_mat > 1 ? rows[0] : total;
     g.s2 = n_mat > 2 ? rows[0] + rows[1] : total;
-    return gemm_enqueue(s, g, x, true, y, m, total, n_cols, dtype, gemm_work(m, total, n_cols, dtype, true), ws,
-                        false, norm_w, eps, false, defer, pending);
+    const GemmWork work = f32_work(m, total, n_cols, dtype, ws_bytes);
+    if (work.total > ws_bytes) return set_error(YULE_ERR_INVALID, "gemm: workspace too small");
+    return gemm_enqueue(s, g, x, true, y, m, total, n_cols, dtype, work, ws, false, norm_w, eps, false, defer, pending);
 }
 
 extern "C" int yule_hip_quantized_gemm(yule_hip_backend *be, yule_buffer weights, yule_buffer x_bf16, yule_buffer y,

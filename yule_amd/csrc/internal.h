@@ -61,12 +61,16 @@ int get_buffer(yule_hip_backend *be, uint64_t h, size_t need, void **ptr, const 
 // until it is destroyed, so a call enqueues every launch that uses the
 // workspace before another thread's call can get it: launches on the one
 // backend stream then never interleave over it.  Growing it waits for the
-// stream (earlier launches may still read the old one).
+// stream (earlier launches may still read the old one); under stream capture
+// it is refused and the capture goes on.
 struct ScratchLease {
     std::unique_lock<std::mutex> lock;
     void *ptr = nullptr;
 };
 int get_scratch(yule_hip_backend *be, size_t need, ScratchLease *lease);
+// device memory for a workspace: YULE_ERR_OOM when the card has no room, or
+// above YULE_WORKSPACE_LIMIT_MB (environment) megabytes in one allocation
+int workspace_alloc(size_t bytes, void **p, const char *what);
 
 // Launch failures surface through hipGetLastError after a kernel launch.
 int check_launch(const char *what);
@@ -155,7 +159,9 @@ size_t attn_chunk_scratch_bytes(uint32_t n_heads, uint32_t hd, uint32_t max_rows
 int launch_attn_chunks(hipStream_t stream, const float *q, const float *kc, const float *vc, const uint32_t *ctl,
                        float *out, void *scratch, uint32_t n_heads, uint32_t n_kv, uint32_t hd, uint32_t max_rows,
                        uint32_t seq_host);
-// f32-X prefill GEMM into a caller-owned workspace (gemm.hip)
+// f32-X prefill GEMM into a caller-owned workspace of ws_bytes (gemm.hip):
+// of the plans, the preferred one that fits runs; *_workspace_bytes are what
+// the preferred one needs, or the one that needs least (least)
 // A split-K reduction left for the next product's X pre-pass (defer): the
 // partials part[ks][m][ny] of y, summed into y (accumulate: added to it) by
 // the pre-pass of the product whose X is y (pending), row by row before it
@@ -168,22 +174,23 @@ struct GemmRed {
     bool accumulate;
 };
 bool gemm_supports(uint32_t dtype, uint32_t n_cols);
-size_t gemm_f32_workspace_bytes(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype);
+size_t gemm_f32_workspace_bytes(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool least = false);
 // up to three matrices of one format sharing X as one f32-X product into
 // Y [m][sum of rows] (each row count a multiple of 256)
 bool gemm_multi_ok(uint32_t dtype, uint32_t n_cols, const uint32_t *rows, uint32_t n_mat);
 size_t gemm_f32_multi_workspace_bytes(uint32_t m, const uint32_t *rows, uint32_t n_mat, uint32_t n_cols,
-                                      uint32_t dtype);
+                                      uint32_t dtype, bool least = false);
 int launch_gemm_f32_multi(hipStream_t stream, const uint8_t *const *w, const uint32_t *rows, uint32_t n_mat,
                           const float *x, float *y, uint32_t m, uint32_t n_cols, uint32_t dtype, void *ws,
-                          const float *norm_w = nullptr, float eps = 0.f, GemmRed *defer = nullptr,
+                          size_t ws_bytes, const float *norm_w = nullptr, float eps = 0.f, GemmRed *defer = nullptr,
                           const GemmRed *pending = nullptr);
 // accumulate: Y += X W (the residual add of the output and down projections);
 // norm_w: X's rows RMS-normalised and scaled by norm_w (eps) on the way in;
 // glu: x holds [gate | up] rows (2 n_cols wide) and X = gate * sigmoid(gate)
 // * up, formed on the way in (the down projection after a gate|up product)
 int launch_gemm_f32(hipStream_t stream, const uint8_t *w, const float *x, float *y, uint32_t m, uint32_t n_rows,
-                    uint32_t n_cols, uint32_t dtype, void *ws, bool accumulate = false, const float *norm_w = nullptr,
+                    uint32_t n_cols, uint32_t dtype, void *ws, size_t ws_bytes, bool accumulate = false,
+                    const float *norm_w = nullptr,
                     float eps = 0.f, bool glu = false, GemmRed *defer = nullptr, const GemmRed *pending = nullptr);
 // batched prompt pass (prefill.hip)
 int launch_embed_rows_batch(hipStream_t stream, uint32_t dtype, const uint8_t *table, const uint32_t *tokens,

@@ -64,6 +64,7 @@ struct yule_hip_runner {
     float *bqkv = nullptr, *bgu = nullptr;
     void *bws = nullptr;
     size_t bws_size = 0;
+    bool bws_least = false;   // the card had no room for the preferred GEMM plans' workspace
     float last_prefill_ms = 0.f;
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -358,19 +359,18 @@ bool gu_one(const yule_hip_runner *r, const yule_hip_runner::Layer &L) {
 }
 
 // GEMM workspace the batched pass over n rows needs (the largest of its
-// products)
-size_t batch_workspace(const yule_hip_runner *r, uint32_t n) {
+// products, as the preferred plans run them or those that need least)
+size_t batch_workspace(const yule_hip_runner *r, uint32_t n, bool least) {
     const uint32_t qd = r->n_heads * r->hd, kvd = r->n_kv * r->hd;
     size_t need = 0;
     for (const auto &L : r->layers) {
-        const size_t w[7] = {gemm_f32_workspace_bytes(n, qd, r->dim, L.tq), gemm_f32_workspace_bytes(n, kvd, r->dim, L.tk),
-                             gemm_f32_workspace_bytes(n, kvd, r->dim, L.tv), gemm_f32_workspace_bytes(n, r->dim, qd, L.to),
-                             gemm_f32_workspace_bytes(n, r->ff, r->dim, L.tg), gemm_f32_workspace_bytes(n, r->ff, r->dim, L.tu),
-                             gemm_f32_workspace_bytes(n, r->dim, r->ff, L.td)};
-        for (size_t v : w) need = std::max(need, v);
+        const struct { uint32_t rows, cols, dtype; } prod[7] = {{qd, r->dim, L.tq}, {kvd, r->dim, L.tk}, {kvd, r->dim, L.tv},
+                                                                {r->dim, qd, L.to}, {r->ff, r->dim, L.tg}, {r->ff, r->dim, L.tu},
+                                                                {r->dim, r->ff, L.td}};
+        for (const auto &p : prod) need = std::max(need, gemm_f32_workspace_bytes(n, p.rows, p.cols, p.dtype, least));
         const uint32_t qkv[3] = {qd, kvd, kvd}, gu[2] = {r->ff, r->ff};
-        if (qkv_one(r, L)) need = std::max(need, gemm_f32_multi_workspace_bytes(n, qkv, 3, r->dim, L.tq));
-        if (gu_one(r, L)) need = std::max(need, gemm_f32_multi_workspace_bytes(n, gu, 2, r->dim, L.tg));
+        if (qkv_one(r, L)) need = std::max(need, gemm_f32_multi_workspace_bytes(n, qkv, 3, r->dim, L.tq, least));
+        if (gu_one(r, L)) need = std::max(need, gemm_f32_multi_workspace_bytes(n, gu, 2, r->dim, L.tg, least));
     }
     return need;
 }
@@ -389,7 +389,8 @@ int ensure_batch(yule_hip_runner *r, uint32_t n) {
     // two workspaces: a product whose split-K reduction is left to the next
     // product's pre-pass keeps its partials in one while the next runs in
     // the other
-    const size_t need = 2 * ((batch_workspace(r, n) + 255) & ~(size_t)255);
+    auto need_of = [&](bool least) { return 2 * ((batch_workspace(r, n, least) + 255) & ~(size_t)255); };
+    size_t need = need_of(r->bws_least);
     if (need > r->bws_size) {
         if (r->bws) {
             if ((rc = hip_error(hipStreamSynchronize(r->be->stream), "runner: synchronize"))) return rc;
@@ -397,7 +398,13 @@ int ensure_batch(yule_hip_runner *r, uint32_t n) {
             r->bws = nullptr;
             r->bws_size = 0;
         }
-        if ((rc = hip_error(hipMalloc(&r->bws, need), "runner: prefill workspace"))) return rc;
+        rc = workspace_alloc(need, &r->bws, "runner: prefill workspace");
+        if (rc && !r->bws_least) {
+            r->bws_least = true;
+            need = need_of(true);
+            rc = workspace_alloc(need, &r->bws, "runner: prefill workspace");
+        }
+        if (rc) return rc;
         r->bws_size = need;
     }
     return YULE_OK;
@@ -423,7 +430,8 @@ int prefill_rows(yule_hip_runner *r, uint32_t pos0, uint32_t n, uint32_t prompt_
     // products leave their split-K reduction to the next product's pre-pass
     // (red), which reads their X right after (except the last down: the head
     // reads its rows)
-    void *wsv[2] = {r->bws, static_cast<uint8_t *>(r->bws) + r->bws_size / 2};
+    const size_t wsn = r->bws_size / 2;
+    void *wsv[2] = {r->bws, static_cast<uint8_t *>(r->bws) + wsn};
     uint32_t wi = 0;
     auto next_ws = [&]() { return wsv[wi ^= 1]; };
     GemmRed red{}, none{};
@@ -437,18 +445,18 @@ int prefill_rows(yule_hip_runner *r, uint32_t pos0, uint32_t n, uint32_t prompt_
         uint32_t ldq = qd, ldkv = kvd;
         if (qkv_one(r, L)) {
             const uint8_t *w[3] = {L.wq, L.wk, L.wv};
-            if ((rc = launch_gemm_f32_multi(s, w, qkv_rows, 3, r->bx, r->bqkv, n, r->dim, L.tq, next_ws(), L.attn_norm,
+            if ((rc = launch_gemm_f32_multi(s, w, qkv_rows, 3, r->bx, r->bqkv, n, r->dim, L.tq, next_ws(), wsn, L.attn_norm,
                                             r->eps, nullptr, &red)))
                 return rc;
             q = r->bqkv;
             k = r->bqkv + qd;
             v = r->bqkv + qd + kvd;
             ldq = ldkv = qd + 2 * kvd;
-        } else if ((rc = launch_gemm_f32(s, L.wq, r->bx, r->bq, n, qd, r->dim, L.tq, next_ws(), false, L.attn_norm,
+        } else if ((rc = launch_gemm_f32(s, L.wq, r->bx, r->bq, n, qd, r->dim, L.tq, next_ws(), wsn, false, L.attn_norm,
                                          r->eps, false, nullptr, &red)) ||
-                   (rc = launch_gemm_f32(s, L.wk, r->bx, r->bk, n, kvd, r->dim, L.tk, next_ws(), false, L.attn_norm,
+                   (rc = launch_gemm_f32(s, L.wk, r->bx, r->bk, n, kvd, r->dim, L.tk, next_ws(), wsn, false, L.attn_norm,
                                          r->eps)) ||
-                   (rc = launch_gemm_f32(s, L.wv, r->bx, r->bv, n, kvd, r->dim, L.tv, next_ws(), false, L.attn_norm,
+                   (rc = launch_gemm_f32(s, L.wv, r->bx, r->bv, n, kvd, r->dim, L.tv, next_ws(), wsn, false, L.attn_norm,
                                          r->eps))) {
             return rc;
         }
@@ -456,7 +464,7 @@ int prefill_rows(yule_hip_runner *r, uint32_t pos0, uint32_t n, uint32_t prompt_
         if ((rc = launch_rope_rows(s, const_cast<float *>(q), k, v, L.kc, L.vc, r->cos_t, r->sin_t, pos0, n, qd, kvd,
                                    r->hd, ldq, ldkv)) ||
             (rc = launch_attn_prefill(s, q, L.kc, L.vc, r->ba, pos0, n, r->n_heads, r->n_kv, r->hd, ldq)) ||
-            (rc = launch_gemm_f32(s, L.wo, r->ba, r->bx, n, r->dim, qd, L.to, next_ws(), true, nullptr, 0.f, false,
+            (rc = launch_gemm_f32(s, L.wo, r->ba, r->bx, n, r->dim, qd, L.to, next_ws(), wsn, true, nullptr, 0.f, false,
                                   &red)))   // residual += O
             return rc;
         // gate and up: one [gate | up] product when they share a format
@@ -466,19 +474,19 @@ int prefill_rows(yule_hip_runner *r, uint32_t pos0, uint32_t n, uint32_t prompt_
         if (gu) {
             const uint8_t *w[2] = {L.wg, L.wu};
             const GemmRed in = red;
-            if ((rc = launch_gemm_f32_multi(s, w, gu_rows, 2, r->bx, r->bgu, n, r->dim, L.tg, next_ws(), L.ffn_norm,
+            if ((rc = launch_gemm_f32_multi(s, w, gu_rows, 2, r->bx, r->bgu, n, r->dim, L.tg, next_ws(), wsn, L.ffn_norm,
                                             r->eps, &red, &in)))
                 return rc;
         } else {
-            if ((rc = launch_gemm_f32(s, L.wg, r->bx, r->bg, n, r->ff, r->dim, L.tg, next_ws(), false, L.ffn_norm, r->eps,
+            if ((rc = launch_gemm_f32(s, L.wg, r->bx, r->bg, n, r->ff, r->dim, L.tg, next_ws(), wsn, false, L.ffn_norm, r->eps,
                                       false, nullptr, &red)) ||
-                (rc = launch_gemm_f32(s, L.wu, r->bx, r->bu, n, r->ff, r->dim, L.tu, next_ws(), false, L.ffn_norm, r->eps)) ||
+                (rc = launch_gemm_f32(s, L.wu, r->bx, r->bu, n, r->ff, r->dim, L.tu, next_ws(), wsn, false, L.ffn_norm, r->eps)) ||
                 (rc = launch_eltwise(s, 3, r->bg, r->bu, r->bg, n * r->ff)))
                 return rc;
             red = none;
         }
         const GemmRed in = red;
-        if ((rc = launch_gemm_f32(s, L.wd, gu ? r->bgu : r->bg, r->bx, n, r->dim, r->ff, L.td, next_ws(), true, nullptr,
+        if ((rc = launch_gemm_f32(s, L.wd, gu ? r->bgu : r->bg, r->bx, n, r->dim, r->ff, L.td, next_ws(), wsn, true, nullptr,
                                   0.f, gu, last ? nullptr : &red, &in)))   // residual += down
             return rc;
         if (last) red = none;

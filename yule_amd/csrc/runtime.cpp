@@ -7,6 +7,7 @@
 // (yule-gpu/src/cpu.rs:157), Result<()> as status code + message.
 #include <atomic>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -27,6 +28,7 @@ int set_error(int code, const std::string &msg) {
 
 int hip_error(hipError_t e, const char *what) {
     if (e == hipSuccess) return YULE_OK;
+    (void)hipGetLastError();   // reported here: the next launch's check does not find it again
     return set_error(e == hipErrorOutOfMemory ? YULE_ERR_OOM : YULE_ERR_HIP,
                      std::string(what) + ": " + hipGetErrorString(e));
 }
@@ -36,10 +38,25 @@ int check_launch(const char *what) {
     return e == hipSuccess ? YULE_OK : hip_error(e, what);
 }
 
+int workspace_alloc(size_t bytes, void **p, const char *what) {
+    const char *e = getenv("YULE_WORKSPACE_LIMIT_MB");
+    const unsigned long long limit = e ? strtoull(e, nullptr, 10) : 0;
+    *p = nullptr;
+    if (limit && bytes > limit << 20)
+        return set_error(YULE_ERR_OOM, std::string(what) + ": " + std::to_string(bytes) +
+                                           " bytes, above YULE_WORKSPACE_LIMIT_MB");
+    return hip_error(hipMalloc(p, bytes), what);
+}
+
 int get_scratch(yule_hip_backend *be, size_t need, ScratchLease *lease) {
     std::unique_lock<std::mutex> lk(be->scratch_mu);
     if (be->scratch_size < need) {
         int rc;
+        // neither the wait nor the allocation can be captured, and trying would spoil the capture
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if ((rc = hip_error(hipStreamIsCapturing(be->stream, &cap), "scratch: capture status"))) return rc;
+        if (cap != hipStreamCaptureStatusNone)
+            return set_error(YULE_ERR_HIP, "scratch: cannot grow under stream capture");
         if (be->scratch) {
             if ((rc = hip_error(hipStreamSynchronize(be->stream), "scratch: synchronize"))) return rc;
             (void)hipFree(be->scratch);
@@ -47,7 +64,7 @@ int get_scratch(yule_hip_backend *be, size_t need, ScratchLease *lease) {
             be->scratch_size = 0;
         }
         const size_t sz = (need + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
-        if ((rc = hip_error(hipMalloc(&be->scratch, sz), "scratch: allocate"))) return rc;
+        if ((rc = workspace_alloc(sz, &be->scratch, "scratch: allocate"))) return rc;
         be->scratch_size = sz;
     }
     lease->ptr = be->scratch;
