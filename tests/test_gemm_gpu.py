@@ -128,6 +128,37 @@ def test_gemm_few_rows_q8_0(hip, M, N, K):
             assert np.max(np.abs(ref)) < 3e38 and np.max(np.abs(got[m] - ref)) <= tolerance_bar(ref), f"row {m}"
 
 
+def rel_error(got, ref):
+    """2-norm of the difference over 2-norm of the result, in f64."""
+    return float(np.linalg.norm(got.astype(np.float64) - ref) / np.linalg.norm(ref))
+
+
+@pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
+def test_gemm_few_rows_q8_0_small_rows(hip, f32):
+    """The one-launch kernel on rows far below 1: as exact as ordinary ones down
+    to the subnormals (f32 sums of 2304 terms: well under 4e-6), alone, beside
+    ordinary rows, a zero row, and a row whose 256-column units differ."""
+    N, K, dt = 96, 2304, DType.Q8_0
+    say(f"[gemm] few rows Q8_0, small rows, {'f32' if f32 else 'bf16'} X")
+    w = synth.gen_quant(dt, 150, N, K)
+    scale = np.float32(2.0) ** np.array([-118, -122, -100, -64, 0, -63, -125, -90, 0], np.float32)
+    x = synth.gauss(151, (9, K)) * scale[:, None]
+    x[8, 256:] *= np.float32(2.0 ** -120)      # one ordinary unit, eight small ones
+    x[7, :] = 0
+    if f32:
+        got = run_gemm_f32(hip, dt, w, x, 9, N, K)
+    else:
+        xb = bf16_bits(x)
+        got, x = run_gemm(hip, dt, w, xb, 9, N, K), bf16_to_f32(xb).reshape(9, K)
+    for m in range(9):
+        ref = oracle.qmv_f64(int(dt), w, np.ascontiguousarray(x[m]), N, K).astype(np.float64)
+        if m == 7:
+            assert not np.any(got[m])
+        else:
+            # results next to the smallest normal f32 carry its spacing, 2^-149
+            assert rel_error(got[m], ref) <= 4e-6 + 2.0 ** -148 * np.sqrt(N) / np.linalg.norm(ref), f"row {m}"
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 77, 1024), (5, 300, 3072), (16, 64, 2048), (17, 129, 1024),
                                    (32, 200, 3072), (32, 1000, 2048), (8, 4096, 5120), (3, 2000, 14336),
                                    (33, 1000, 2048)])

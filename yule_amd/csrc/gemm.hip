@@ -1597,7 +1597,8 @@ static void *static_workspace(int device) {
 // (rows = X rows, columns = weight rows, so a lane's block scale is its own
 // row's), scaled into f32 accumulators that meet in LDS.  Quants are exact in
 // bf16 and f32 X is the exact sum of three bf16 parts, so only the f32 sums
-// round.  Bound by the address work of its 8-byte weight reads and of X, which
+// round: a unit of an X row whose magnitudes are all below 2^-64 is raised by
+// 2^96 first, so that no part and no product nears the subnormals.  Bound by the address work of its 8-byte weight reads and of X, which
 // every workgroup reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
 // reduction -> this): 256x1024 15.6 -> 4.6, 1030x2048 17.0 -> 8.9, 4096x4096
 // 26.4 -> 17.1 (bf16 X 20.6 -> 13.8; one row of f32 X 25.2 -> 13.3).  Larger
@@ -1605,6 +1606,7 @@ static void *static_workspace(int device) {
 // 4096 f32 X 49.0 there and 53.1 here, bf16 X 30.1 and 45.2.
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef float few_f4 __attribute__((ext_vector_type(4)));
+typedef uint16_t few_us2 __attribute__((ext_vector_type(2)));
 constexpr uint32_t kFewRows = 16;
 constexpr uint64_t kFewWeights = 1ull << 24;   // n_rows * n_cols
 
@@ -1614,6 +1616,7 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
                                                             uint32_t n_cols) {
     constexpr uint32_t NW = 16, U = 8;
     constexpr float kDown = 0x1p-12f;   // quants reach 2^7 and a block sums 2^5: its sum stays within the largest |x|
+    constexpr float kSmall = 0x1p-64f, kUp = 0x1p96f;
     __shared__ __align__(16) float red[NW][256];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), n0 = blockIdx.x * 16;
@@ -1639,6 +1642,50 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
                 xr[b] = *reinterpret_cast<const float4 *>(xh + u * 256 + b * 32);
             }
         }
+        // the row's largest magnitude in this unit: of the lane's values, then
+        // of the row's four lanes
+        float am = 0.f;
+        if constexpr (F32) {
+#pragma unroll
+            for (uint32_t i = 0; i < 2 * U; i++)
+                am = fmaxf(fmaxf(am, fmaxf(fabsf(xr[i].x), fabsf(xr[i].y))), fmaxf(fabsf(xr[i].z), fabsf(xr[i].w)));
+        } else {
+            few_us2 a = {0, 0};   // bf16 magnitudes compare as integers
+#pragma unroll
+            for (uint32_t i = 0; i < U; i++) {
+                uint32_t h[4];
+                __builtin_memcpy(h, &xr[i], 16);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++)
+                    a = __builtin_elementwise_max(a, __builtin_bit_cast(few_us2, h[j] & 0x7FFF7FFFu));
+            }
+            am = __uint_as_float((uint32_t)(a.x > a.y ? a.x : a.y) << 16);
+        }
+        am = fmaxf(am, __shfl_xor(am, 16, 64));
+        am = fmaxf(am, __shfl_xor(am, 32, 64));
+        const bool small = am < kSmall;
+        float back[4] = {1.f / kDown, 1.f / kDown, 1.f / kDown, 1.f / kDown};   // to Y's units, of rows 4 g + r
+        if (__any(small)) {
+            const float up = small ? kUp : 1.f;
+#pragma unroll
+            for (uint32_t i = 0; i < (F32 ? 2 * U : U); i++) {
+                if constexpr (F32) {
+                    xr[i].x *= up; xr[i].y *= up; xr[i].z *= up; xr[i].w *= up;
+                } else {
+                    uint32_t h[4];
+                    __builtin_memcpy(h, &xr[i], 16);
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; j++)
+                        h[j] = __builtin_amdgcn_perm(__float_as_uint(__uint_as_float(h[j] & 0xFFFF0000u) * up),
+                                                     __float_as_uint(__uint_as_float(h[j] << 16) * up), 0x07060302u);
+                    __builtin_memcpy(&xr[i], h, 16);
+                }
+            }
+            const float d = small ? 1.f / kDown / kUp : 1.f / kDown;
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) back[r] = __shfl(d, (int)(4 * g + r), 64);
+        }
+        few_f4 sum = {0, 0, 0, 0};
 #pragma unroll
         for (uint32_t b = 0; b < U; b++) {
             // X as bf16 parts (one, or three that sum to the f32 exactly)
@@ -1678,8 +1725,10 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
             __builtin_memcpy(&d, &ds[b], 2);
             const float df = (float)d;
 #pragma unroll
-            for (uint32_t r = 0; r < 4; r++) acc[r] += df * t[r];
+            for (uint32_t r = 0; r < 4; r++) sum[r] += df * t[r];
         }
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) acc[r] += back[r] * sum[r];
     }
     *reinterpret_cast<few_f4 *>(&red[wave][4 * lane]) = acc;
     __syncthreads();
@@ -1688,7 +1737,7 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
     float sum = 0.f;
 #pragma unroll
     for (uint32_t i = 0; i < NW; i++) sum += red[i][4 * ((om >> 2) * 16 + on) + (om & 3u)];
-    y[(size_t)om * n_rows + row] = sum * (1.0f / kDown);
+    y[(size_t)om * n_rows + row] = sum;
 }
 
 static int launch_gemm_few_q80(hipStream_t s, const uint8_t *w, const void *x, bool f32x, float *y, uint32_t m,
