@@ -204,9 +204,18 @@ def test_gqa_decode_attn_long(hip, hd, nh, nkv, seq):
 @pytest.mark.parametrize("hd,nh,nkv,seq", [(64, 8, 8, 20481), (128, 8, 8, 12097), (128, 16, 2, 82001),
                                           (64, 48, 16, 7937), (128, 32, 32, 2033)])
 def test_gqa_decode_attn_chunk_lengths(hip, hd, nh, nkv, seq):
-    """Split-KV chunks of 320, 192, 320, 256 and 128 positions with a short
-    last chunk (one key, or part of a 16-key sub-tile)."""
+    """Split-KV chunks with a short last one (one key, or part of a 16-key
+    sub-tile): the tile kernel's of 320, 256 and 256 positions (first, third
+    and fourth case), the vector kernel's of 128."""
     say(f"[ops] gqa_decode_attn chunks hd={hd} heads={nh}/{nkv} seq={seq}")
+    run_gqa_case(hip, hd, nh, nkv, seq)
+
+
+@pytest.mark.parametrize("hd,nh,nkv,seq", [(64, 32, 32, 513), (64, 32, 32, 3840), (64, 32, 32, 3841), (128, 8, 8, 16129)])
+def test_gqa_decode_attn_one_query_head(hip, hd, nh, nkv, seq):
+    """One query head per KV head: the vector kernel up to the length at which
+    its chunks would be 256 long, the tile kernel from there on."""
+    say(f"[ops] one query head per KV head, hd={hd} heads={nh}/{nkv} seq={seq}")
     run_gqa_case(hip, hd, nh, nkv, seq)
 
 

@@ -1904,6 +1904,19 @@ size_t split_scratch_bytes(uint32_t n_heads, uint32_t hd, uint32_t seq_cap) {
     return (size_t)n_heads * mc * hd * sizeof(float) + (size_t)n_heads * mc * sizeof(float2) + 256;
 }
 
+// The tile kernel or the vector one (attn_split_kernel).  With one query head
+// per KV head fifteen of a tile's sixteen columns repeat it, and the vector
+// kernel is ahead until its chunks are 256 long; vector / tile, us (both with
+// the combine): 16 heads x 128: 1615 positions 9.1 / 10.2, 4500 17.5 / 19.6,
+// 11000 70.7 / 32.9; 32 x 64: 1615 9.0 / 10.2, 3300 15.1 / 15.5, 4500 22.6 /
+// 20.0; 8 x 128: 3300 8.9 / 10.3, 11000 21.6 / 21.5.  With two and more the
+// tile kernel is level (16/8 x 128: 1000 9.7 / 9.1, 3300 10.6 / 11.2) to far
+// ahead (12/2 x 128, 3300: 12.4 / 8.8).  A decode step's launch serves every
+// position up to seq_cap and goes by that.
+static bool split_tile_ok(uint32_t n_heads, uint32_t n_kv, uint32_t hd, uint32_t seq_cap) {
+    return (hd == 64 || hd == 128) && (n_heads > n_kv || split_chunk(seq_cap, n_kv) == 256);
+}
+
 int launch_attn_split(hipStream_t s, const float *q, const float *k, const float *v, float *kc, float *vc,
                       const float *cos_t, const float *sin_t, const uint32_t *ctl, float *out, void *scratch,
                       uint32_t n_heads, uint32_t n_kv, uint32_t hd, uint32_t seq_cap) {
@@ -1912,9 +1925,9 @@ int launch_attn_split(hipStream_t s, const float *q, const float *k, const float
     float *part = static_cast<float *>(scratch);
     float2 *ml = reinterpret_cast<float2 *>(part + (size_t)n_heads * mc * hd);
     const uint32_t seq_host = ctl ? 0u : seq_cap;
-    const bool tile = hd == 64 || hd == 128;
+    const bool tile = split_tile_ok(n_heads, n_kv, hd, seq_cap);
     const uint32_t C = tile ? split_tile_chunk(seq_cap, n_kv) : split_chunk(seq_cap, n_kv);
-        const dim3 grid(n_kv, ctl ? mc : (seq_cap + C - 1) / C);
+    const dim3 grid(n_kv, ctl ? mc : (seq_cap + C - 1) / C);
 #define YULE_SPLIT_ARGS q, k, v, kc, vc, cos_t, sin_t, ctl, part, ml
 #define YULE_SPLIT_CASE(G)                                                                                       \
     case G:                                                                                                      \
@@ -1923,9 +1936,9 @@ int launch_attn_split(hipStream_t s, const float *q, const float *k, const float
     const uint32_t group = n_heads / n_kv;
     if (!group || group > kSplitMaxGroup)
         return set_error(YULE_ERR_UNSUPPORTED, "split attention: more than 8 query heads per KV head");
-    if (hd == 64)
+    if (tile && hd == 64)
         hipLaunchKernelGGL(attn_split_tile_kernel<64>, grid, dim3(256), 0, s, YULE_SPLIT_ARGS, group, n_kv, seq_host, mc);
-    else if (hd == 128)
+    else if (tile)
         hipLaunchKernelGGL(attn_split_tile_kernel<128>, grid, dim3(256), 0, s, YULE_SPLIT_ARGS, group, n_kv, seq_host, mc);
     else
         switch (group) {
