@@ -219,6 +219,15 @@ def test_gqa_decode_attn_one_query_head(hip, hd, nh, nkv, seq):
     run_gqa_case(hip, hd, nh, nkv, seq)
 
 
+@pytest.mark.parametrize("hd,nh,nkv,seq", [(128, 16, 8, 12097), (64, 32, 8, 20481), (128, 24, 12, 12033), (64, 12, 4, 16385)])
+def test_gqa_decode_attn_row_lengths(hip, hd, nh, nkv, seq):
+    """The tile kernel's chunks by the length of a cache row: 192 and 320
+    positions for 4096 and 2048 bytes, 256 and 128 for others, each with a
+    short last chunk."""
+    say(f"[ops] gqa_decode_attn rows of {4 * nkv * hd} bytes, seq={seq}")
+    run_gqa_case(hip, hd, nh, nkv, seq)
+
+
 def test_gqa_decode_attn_limits(hip):
     """More than 8 query heads per KV head: the per-head kernel up to 16384
     positions, refused above; above 262144 positions refused for any shape."""

@@ -1115,17 +1115,17 @@ __host__ __device__ inline uint32_t split_chunk(uint32_t seq, uint32_t n_kv) {
     return 64;
 }
 
-// The same for attn_split_tile_kernel.  Below 16 KV heads the chunks are 192
-// and 320 long: workgroups in flight start a chunk of rows apart, and with
-// 4096-byte rows (8 heads of 128) a power of two puts them on the same memory
-// channels.  32/8 heads x 128, 15001 positions: 192 22.1 us, 128 28.4, 256
-// 28.8; 60000 positions: 320 81.8, 256 91.2, 128 101.9 (and the combine 5.8
-// against 10.1).  A position of 16 or more heads covers the channels by
-// itself, and 128 fills the chip earlier (32 heads x 128, 2000 positions: 128
-// 11.8 us, 192 15.0).
-__host__ __device__ inline uint32_t split_tile_chunk(uint32_t seq, uint32_t n_kv) {
-    if (n_kv >= 16) return split_chunk(seq, n_kv);
-    const uint32_t target = 512;
+// The same for attn_split_tile_kernel.  Rows of 2048 or 4096 bytes (below 16
+// KV heads) take chunks of 192 and 320: workgroups in flight start a chunk of
+// rows apart, and a power of two puts them on the same memory channels.  Call
+// with those chunks against split_chunk's, us: 8 heads x 128, 15001 positions
+// 26.7 / 28.8, 25000 39.3 / 44.6; 8 x 64, 25000 23.7 / 24.5; 4 x 128, 60000
+// 42.9 / 45.8.  Other row lengths meet the channels out of step by themselves
+// and only lose by them: 12 x 128, 15001 38.4 / 34.0; 12 x 64, 15001 23.8 /
+// 21.6; 2 x 128, 40000 27.0 / 24.1; 4 x 64, 25000 17.3 / 16.4.
+__host__ __device__ inline uint32_t split_tile_chunk(uint32_t seq, uint32_t n_kv, uint32_t hd) {
+    const uint32_t row = 4 * n_kv * hd, target = 512;
+    if (n_kv >= 16 || (row != 2048 && row != 4096)) return split_chunk(seq, n_kv);
     if (n_kv * ((seq + 319) / 320) >= target) return 320;
     if (n_kv * ((seq + 191) / 192) >= target) return 192;
     return 64;
@@ -1296,7 +1296,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), kvh = blockIdx.x, chunk = blockIdx.y;
     const bool step = ctl != nullptr;
     const uint32_t seq = step ? ctl[0] + 1 : seq_host, pos = seq - 1;
-    const uint32_t C = split_tile_chunk(seq, n_kv), c0 = chunk * C;
+    const uint32_t C = split_tile_chunk(seq, n_kv, HD), c0 = chunk * C;
     if (c0 >= seq) return;   // uniform over the workgroup
     const uint32_t end = c0 + C < seq ? c0 + C : seq, h0 = kvh * G;
     T st;
@@ -1423,7 +1423,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restri
     __shared__ float4 os[256];
     const uint32_t h = blockIdx.x, tid = threadIdx.x;
     const uint32_t seq = ctl ? ctl[0] + 1 : seq_host;
-    const uint32_t C = BASE2 ? split_tile_chunk(seq, n_kv) : split_chunk(seq, n_kv), n_ch = (seq + C - 1) / C;
+    const uint32_t C = BASE2 ? split_tile_chunk(seq, n_kv, hd) : split_chunk(seq, n_kv), n_ch = (seq + C - 1) / C;
     const float2 *mh = ml + (size_t)h * max_chunks;
     float mx = -INFINITY;
     for (uint32_t c = tid; c < n_ch; c += 256) mx = fmaxf(mx, mh[c].x);
@@ -1926,7 +1926,7 @@ int launch_attn_split(hipStream_t s, const float *q, const float *k, const float
     float2 *ml = reinterpret_cast<float2 *>(part + (size_t)n_heads * mc * hd);
     const uint32_t seq_host = ctl ? 0u : seq_cap;
     const bool tile = split_tile_ok(n_heads, n_kv, hd, seq_cap);
-    const uint32_t C = tile ? split_tile_chunk(seq_cap, n_kv) : split_chunk(seq_cap, n_kv);
+    const uint32_t C = tile ? split_tile_chunk(seq_cap, n_kv, hd) : split_chunk(seq_cap, n_kv);
     const dim3 grid(n_kv, ctl ? mc : (seq_cap + C - 1) / C);
 #define YULE_SPLIT_ARGS q, k, v, kc, vc, cos_t, sin_t, ctl, part, ml
 #define YULE_SPLIT_CASE(G)                                                                                       \
