@@ -1597,7 +1597,7 @@ static void *static_workspace(int device) {
 // (rows = X rows, columns = weight rows, so a lane's block scale is its own
 // row's), scaled into f32 accumulators that meet in LDS.  Quants are exact in
 // bf16 and f32 X is the exact sum of three bf16 parts, so only the f32 sums
-// round: a unit of an X row whose magnitudes are all below 2^-64 is raised by
+// round: a unit of an X row whose magnitudes are all below 2^-63 is raised by
 // 2^96 first, so that no part and no product nears the subnormals.  Bound by the address work of its 8-byte weight reads and of X, which
 // every workgroup reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
 // reduction -> this): 256x1024 15.6 -> 4.6, 1030x2048 17.0 -> 8.9, 4096x4096
@@ -1606,7 +1606,6 @@ static void *static_workspace(int device) {
 // 4096 f32 X 49.0 there and 53.1 here, bf16 X 30.1 and 45.2.
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef float few_f4 __attribute__((ext_vector_type(4)));
-typedef uint16_t few_us2 __attribute__((ext_vector_type(2)));
 constexpr uint32_t kFewRows = 16;
 constexpr uint64_t kFewWeights = 1ull << 24;   // n_rows * n_cols
 
@@ -1616,7 +1615,7 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
                                                             uint32_t n_cols) {
     constexpr uint32_t NW = 16, U = 8;
     constexpr float kDown = 0x1p-12f;   // quants reach 2^7 and a block sums 2^5: its sum stays within the largest |x|
-    constexpr float kSmall = 0x1p-64f, kUp = 0x1p96f;
+    constexpr float kUp = 0x1p96f;
     __shared__ __align__(16) float red[NW][256];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), n0 = blockIdx.x * 16;
@@ -1624,8 +1623,10 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
     const uint8_t *wr = w + (size_t)(n0 + c < n_rows ? n0 + c : n_rows - 1) * (n_cols / 32) * 34;
     const float *xf = static_cast<const float *>(xv) + (size_t)mr * n_cols + 8 * g;
     const uint16_t *xh = static_cast<const uint16_t *>(xv) + (size_t)mr * n_cols + 8 * g;
-    few_f4 acc = {0, 0, 0, 0};
-    for (uint32_t u = wave; u < n_cols / 256; u += NW) {
+    // one unit of 256 columns: the sums of the lane's column and rows 4 g + r.
+    // raise (wave-uniform): the rows in the bits of `small` times kUp first.
+    // top: the OR of the lane's X bits
+    auto unit = [&](uint32_t u, auto raise, uint32_t small, uint32_t &top) {
         uint2 qs[U];
         uint16_t ds[U];
         float4 xr[F32 ? 2 * U : U];
@@ -1642,58 +1643,24 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
                 xr[b] = *reinterpret_cast<const float4 *>(xh + u * 256 + b * 32);
             }
         }
-        // the row's largest magnitude in this unit: of the lane's values, then
-        // of the row's four lanes
-        float am = 0.f;
-        if constexpr (F32) {
-#pragma unroll
-            for (uint32_t i = 0; i < 2 * U; i++)
-                am = fmaxf(fmaxf(am, fmaxf(fabsf(xr[i].x), fabsf(xr[i].y))), fmaxf(fabsf(xr[i].z), fabsf(xr[i].w)));
-        } else {
-            few_us2 a = {0, 0};   // bf16 magnitudes compare as integers
-#pragma unroll
-            for (uint32_t i = 0; i < U; i++) {
-                uint32_t h[4];
-                __builtin_memcpy(h, &xr[i], 16);
-#pragma unroll
-                for (uint32_t j = 0; j < 4; j++)
-                    a = __builtin_elementwise_max(a, __builtin_bit_cast(few_us2, h[j] & 0x7FFF7FFFu));
-            }
-            am = __uint_as_float((uint32_t)(a.x > a.y ? a.x : a.y) << 16);
-        }
-        am = fmaxf(am, __shfl_xor(am, 16, 64));
-        am = fmaxf(am, __shfl_xor(am, 32, 64));
-        const bool small = am < kSmall;
-        float back[4] = {1.f / kDown, 1.f / kDown, 1.f / kDown, 1.f / kDown};   // to Y's units, of rows 4 g + r
-        if (__any(small)) {
-            const float up = small ? kUp : 1.f;
-#pragma unroll
-            for (uint32_t i = 0; i < (F32 ? 2 * U : U); i++) {
-                if constexpr (F32) {
-                    xr[i].x *= up; xr[i].y *= up; xr[i].z *= up; xr[i].w *= up;
-                } else {
-                    uint32_t h[4];
-                    __builtin_memcpy(h, &xr[i], 16);
-#pragma unroll
-                    for (uint32_t j = 0; j < 4; j++)
-                        h[j] = __builtin_amdgcn_perm(__float_as_uint(__uint_as_float(h[j] & 0xFFFF0000u) * up),
-                                                     __float_as_uint(__uint_as_float(h[j] << 16) * up), 0x07060302u);
-                    __builtin_memcpy(&xr[i], h, 16);
-                }
-            }
-            const float d = small ? 1.f / kDown / kUp : 1.f / kDown;
-#pragma unroll
-            for (uint32_t r = 0; r < 4; r++) back[r] = __shfl(d, (int)(4 * g + r), 64);
-        }
+        const float up = (small >> c) & 1u ? kUp : 1.f;
         few_f4 sum = {0, 0, 0, 0};
 #pragma unroll
         for (uint32_t b = 0; b < U; b++) {
             // X as bf16 parts (one, or three that sum to the f32 exactly)
             constexpr uint32_t NP = F32 ? 3 : 1;
             bf8v a[NP];
+            uint32_t xb[F32 ? 8 : 4];
+            __builtin_memcpy(xb, &xr[F32 ? 2 * b : b], sizeof(xb));
+#pragma unroll
+            for (uint32_t i = 0; i < (F32 ? 8 : 4); i++) top |= xb[i];
             if constexpr (F32) {
                 float x[8] = {xr[2 * b].x,     xr[2 * b].y,     xr[2 * b].z,     xr[2 * b].w,
                               xr[2 * b + 1].x, xr[2 * b + 1].y, xr[2 * b + 1].z, xr[2 * b + 1].w};
+                if constexpr (decltype(raise)::value) {
+#pragma unroll
+                    for (uint32_t i = 0; i < 8; i++) x[i] *= up;
+                }
 #pragma unroll
                 for (uint32_t part = 0; part < NP; part++) {
                     uint32_t h[4];
@@ -1706,7 +1673,13 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
                     for (uint32_t i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
                 }
             } else {
-                __builtin_memcpy(&a[0], &xr[b], 16);
+                if constexpr (decltype(raise)::value) {
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; i++)
+                        xb[i] = __builtin_amdgcn_perm(__float_as_uint(__uint_as_float(xb[i] & 0xFFFF0000u) * up),
+                                                      __float_as_uint(__uint_as_float(xb[i] << 16) * up), 0x07060302u);
+                }
+                __builtin_memcpy(&a[0], xb, 16);
             }
             uint32_t wq[4];
 #pragma unroll
@@ -1727,8 +1700,37 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
 #pragma unroll
             for (uint32_t r = 0; r < 4; r++) sum[r] += df * t[r];
         }
+        return sum;
+    };
+    few_f4 acc = {0, 0, 0, 0};
+    bool again = false;
+    // rows whose values in a unit are all below 2^-63 (the two top bits of
+    // every exponent are 0) and not all zero: left to the loop after
+    auto low_rows = [&](uint32_t top) {
+        const uint64_t low = __ballot(!(top & (F32 ? 0x60000000u : 0x60006000u))), any = __ballot(top != 0);
+        return (uint32_t)(low & (low >> 16) & (low >> 32) & (low >> 48) & (any | any >> 16 | any >> 32 | any >> 48)) & 0xFFFFu;
+    };
+    for (uint32_t u = wave; u < n_cols / 256; u += NW) {
+        uint32_t top = 0;
+        const few_f4 sum = unit(u, std::false_type{}, 0u, top);
+        const uint32_t small = low_rows(top);
+        again |= small != 0;
 #pragma unroll
-        for (uint32_t r = 0; r < 4; r++) acc[r] += back[r] * sum[r];
+        for (uint32_t r = 0; r < 4; r++) acc[r] += (small >> (4 * g + r)) & 1u ? 0.f : sum[r] * (1.f / kDown);
+    }
+    if (again) {
+        for (uint32_t u = wave; u < n_cols / 256; u += NW) {
+            uint32_t top = 0;
+            for (uint32_t b = 0; b < U; b++)
+                for (uint32_t i = 0; i < (F32 ? 8 : 4); i++)
+                    top |= F32 ? __float_as_uint(xf[u * 256 + b * 32 + i])
+                               : reinterpret_cast<const uint32_t *>(xh + u * 256 + b * 32)[i];
+            const uint32_t small = low_rows(top);
+            if (!small) continue;
+            const few_f4 sum = unit(u, std::true_type{}, small, top);
+#pragma unroll
+            for (uint32_t r = 0; r < 4; r++) acc[r] += (small >> (4 * g + r)) & 1u ? sum[r] * (1.f / kDown / kUp) : 0.f;
+        }
     }
     *reinterpret_cast<few_f4 *>(&red[wave][4 * lane]) = acc;
     __syncthreads();
