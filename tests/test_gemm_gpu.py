@@ -107,11 +107,11 @@ def test_gemm_wide_tiles(hip, dt, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(1, 1, 256), (13, 77, 2304), (16, 200, 4096), (5, 33, 8448), (16, 4096, 4096),
                                    (17, 200, 4096)])
 def test_gemm_few_rows_q8_0(hip, M, N, K):
-    """Q8_0, M <= 16 on weights of up to 2^24 elements: the one-launch kernel
-    (one unit for one wave, nine and 33 units over 16 waves, a ragged last
-    tile), bf16 and f32 X, every row vs the oracle; f32 X spread over 60 powers
-    of two and a row near the top of the range, whose outputs are finite;
-    M = 17 is the tile kernel's again."""
+    """Q8_0, M <= 16: the one-launch kernel (one unit for one wave, nine units
+    over 16 waves, a ragged last tile), bf16 and f32 X, every row vs the
+    oracle; f32 X spread over 60 powers of two and a row near the top of the
+    range, whose outputs are finite; M = 17 and 8448 columns are the tile
+    kernel's."""
     dt = DType.Q8_0
     say(f"[gemm] few rows Q8_0 M={M} N={N} K={K}")
     w = synth.gen_quant(dt, 130 + M, N, K)
@@ -126,6 +126,24 @@ def test_gemm_few_rows_q8_0(hip, M, N, K):
         for got, x in ((y, xf), (y32, x32)):
             ref = oracle.qmv_f64(int(dt), w, x[m], N, K)
             assert np.max(np.abs(ref)) < 3e38 and np.max(np.abs(got[m] - ref)) <= tolerance_bar(ref), f"row {m}"
+
+
+@pytest.mark.parametrize("N,K", [(40, 5632), (4096, 5632), (4097, 5632), (4097, 2816), (8193, 1792), (16384, 1280), (16385, 256),
+                                 (100, 5888)])
+@pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
+def test_gemm_few_rows_q8_0_line(hip, N, K, f32):
+    """Either side of the line between the one-launch kernel and the tiles (one,
+    two, three, four and five rounds of workgroups; 22 units over 16 waves)."""
+    dt, M = DType.Q8_0, 3
+    say(f"[gemm] few rows Q8_0 {N}x{K} {'f32' if f32 else 'bf16'} X")
+    w, x = synth.gen_quant(dt, 160, N, K), synth.gauss(161 + K, (M, K))
+    if f32:
+        got = run_gemm_f32(hip, dt, w, x, M, N, K)
+    else:
+        xb = bf16_bits(x)
+        got, x = run_gemm(hip, dt, w, xb, M, N, K), bf16_to_f32(xb).reshape(M, K)
+    for m in range(M):
+        assert rel_error(got[m], oracle.qmv_f64(int(dt), w, np.ascontiguousarray(x[m]), N, K)) <= 4e-6, f"row {m}"
 
 
 def rel_error(got, ref):

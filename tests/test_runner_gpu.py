@@ -562,3 +562,21 @@ def test_runner_prefill_attention_tiles(hip, hd, heads, kv, pieces):
             assert np.max(np.abs(got - want)) <= tolerance_bar(want), f"after {at} tokens"
     finally:
         run.close()
+
+
+@pytest.mark.parametrize("hd,heads", [(64, 8), (128, 4)])
+def test_runner_split_one_query_head(hip, hd, heads, monkeypatch):
+    """Split-KV decode steps of a model with one query head per KV head (the
+    vector kernel, rotating q and k and writing the row), from position 19 on."""
+    from yule_amd.model import LlamaConfig
+    monkeypatch.setenv("YULE_ATTN_SPLIT_MIN", "20")
+    m = SyntheticModel.generate(LlamaConfig(n_layers=2, dim=512, n_heads=heads, n_kv_heads=heads, ff_dim=512, vocab=512,
+                                            max_seq=160), seed=24)
+    say(f"[runner] split steps, {heads}/{heads} heads of {hd}")
+    run, ref = HipRunner(hip, m), oracle.Runner(m, n_threads=4)
+    toks = synth.uniform_tokens(34, 140, m.cfg.vocab)
+    for i, t in enumerate(toks):
+        got, want = run.decode_step(int(t)), ref.forward(int(t))
+        if i in (18, 19, 63, 64, 65, 139):
+            assert np.max(np.abs(got - want)) <= tolerance_bar(want), f"position {i}"
+    run.close()

@@ -1600,14 +1600,29 @@ static void *static_workspace(int device) {
 // round: a unit of an X row whose magnitudes are all below 2^-63 is raised by
 // 2^96 first, so that no part and no product nears the subnormals.  Bound by the address work of its 8-byte weight reads and of X, which
 // every workgroup reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
-// reduction -> this): 256x1024 15.6 -> 4.6, 1030x2048 17.0 -> 8.9, 4096x4096
-// 26.4 -> 17.1 (bf16 X 20.6 -> 13.8; one row of f32 X 25.2 -> 13.3).  Larger
-// weights stay on the tiles, which read them in whole lines: 16 rows, 14336 x
-// 4096 f32 X 49.0 there and 53.1 here, bf16 X 30.1 and 45.2.
+// reduction -> this): 256x1024 14.6 -> 4.9, 4096x4096 24.5 -> 16.4 (bf16 X 19.5
+// -> 13.3; one row of f32 X 22.4 -> 12.9).
+//
+// A workgroup's time grows with its columns (16 rows of f32 X: 4096 17.7,
+// 8192 34, 14336 57), the launch's with the rounds that its workgroups take on
+// the CUs; the tiles split long K and read weights in whole lines.  One and 16
+// rows of X, tiles -> this, us:
+//   one round   4096 x 5632   f32 30.0 -> 13.9, 32.0 -> 19.3   bf16 21.5 -> 11.5, 23.6 -> 13.8
+//               512 x 5632    f32 20.0 -> 13.4, 22.4 -> 19.0   bf16 16.1 -> 11.3, 18.4 -> 13.5
+//               512 x 6144    f32 20.7 -> 18.3, 23.2 -> 25.9   bf16 16.7 -> 16.2, 19.5 -> 20.1
+//               512 x 14336   f32 30.4 -> 39.2, 35.3 -> 56.9   bf16 26.2 -> 35.1, 30.7 -> 44.1
+//   two         8192 x 2816   f32 25.1 -> 15.3, 26.9 -> 20.5   bf16 18.1 -> 12.3, 20.8 -> 14.6
+//               5632 x 4096   f32 29.2 -> 25.2, 30.7 -> 35.5   bf16 19.9 -> 21.9, 21.7 -> 27.1
+//   four        16384 x 1280  f32 23.6 -> 18.8, 25.6 -> 24.2   bf16 16.5 -> 13.1, 19.3 -> 15.4
+//   eight       32768 x 512   f32 18.1 -> 22.4, 19.1 -> 27.6   bf16 12.3 -> 16.1, 13.4 -> 18.6
+constexpr uint32_t kFewRows = 16, kFewRounds = 4, kFewCols = 5632;
+static bool few_q80_ok(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype) {
+    const uint32_t rounds = (n_rows / 16 + (n_rows % 16 != 0) + (uint32_t)device_cus() - 1) / (uint32_t)device_cus();
+    return dtype == YULE_DTYPE_Q8_0 && m <= kFewRows && rounds <= kFewRounds && (uint64_t)rounds * n_cols <= kFewCols;
+}
+
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef float few_f4 __attribute__((ext_vector_type(4)));
-constexpr uint32_t kFewRows = 16;
-constexpr uint64_t kFewWeights = 1ull << 24;   // n_rows * n_cols
 
 template <bool F32>
 __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__restrict__ w, const void *__restrict__ xv,
@@ -1769,7 +1784,7 @@ static int gemm_entry(yule_hip_backend *be, yule_buffer weights, yule_buffer x, 
     if (weights == y || weights == x) return set_error(YULE_ERR_INVALID, std::string(what) + ": weights alias x or y");
     if (!m || !n_rows) return YULE_OK;
     if (!n_cols) return launch_fill(be->stream, (float *)py, 0.f, (uint64_t)m * n_rows);
-    const bool few = dtype == YULE_DTYPE_Q8_0 && m <= kFewRows && (uint64_t)n_rows * n_cols <= kFewWeights;
+    const bool few = few_q80_ok(m, n_rows, n_cols, dtype);
     GemmWork g = gemm_work(m, n_rows, n_cols, dtype, f32x, !noalloc);
     if (noalloc) {
         if (g.total > kStaticWorkspaceBytes) g = gemm_work(m, n_rows, n_cols, dtype, f32x, false, true);
