@@ -47,6 +47,23 @@ int main() {
 }
 """
 
+# the tests' wide products: bytes of tail partials and passes, on the 256 CUs of the target
+TAILS = r"""
+#include <cstdio>
+#include "gemm_tiled.h"
+using namespace yule;
+int main() {
+    const uint32_t c[][5] = {CASES};
+    for (auto &x : c) {
+        TiledPlan p;
+        if (!gemm_tiled_plan(x[1], x[2], x[3], x[0], x[4], &p)) { printf("none "); continue; }
+        printf("%zu:%u ", p.t_bytes, (x[2] + p.n_chunk - 1) / p.n_chunk);
+    }
+    printf("\n");
+    return 0;
+}
+"""
+
 
 @pytest.fixture(scope="module")
 def host_run(tmp_path_factory):
@@ -68,6 +85,19 @@ def host_run(tmp_path_factory):
 def test_scale_rows_stay_inside_the_scales(host_run):
     r = host_run("scales", SCALE_WALK, YULE_GEMM_TILED_MIN="1")
     assert r.returncode == 0 and r.stdout.count(".") >= 35, r.stdout + r.stderr
+
+
+def test_wide_cases_have_tail_tiles(host_run):
+    """The shapes that stand for the tail tiles (gemm_tiled_check.py's of 1024
+    and 1536 columns, test_runner_prefill_tail_tiles's output product) have
+    some, in one pass and in two."""
+    from gemm_tiled_check import WIDE
+    from yule_amd import DType
+    cases = [(int(dt), m, n, k, 1) for dt, m, n, k in WIDE if k in (1024, 1536)] + [(int(DType.Q4_K), 2100, 8192, 8192, 1)]
+    r = host_run("tails", TAILS.replace("CASES", ", ".join("{%d, %d, %d, %d, %d}" % c for c in cases)), YULE_GEMM_TILED_MIN="1")
+    got = [tuple(int(v) for v in w.split(":")) for w in r.stdout.split()]
+    assert len(got) == len(cases) == 4 and all(t > 0 for t, _ in got), r.stdout + r.stderr
+    assert [n for _, n in got] == [1, 1, 2, 1]
 
 
 def test_wait_state_between_m0_and_lds_loads():

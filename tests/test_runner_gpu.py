@@ -407,6 +407,40 @@ def test_runner_prefill_batched_forced_splits(hip, splits):
     say(f"[runner] {r.stdout.strip()}")
 
 
+def test_runner_prefill_batched_operand_tiles(hip):
+    """The batched prefill with every projection through the operand tiles
+    (tests/prefill_tiled_check.py, in a child process because the switch is
+    read once per process)."""
+    import os
+    import subprocess
+    say("[runner] batched prefill over operand tiles")
+    r = subprocess.run([sys.executable, "-u", str(Path(__file__).with_name("prefill_tiled_check.py"))],
+                       env=dict(os.environ, YULE_GEMM_TILED_MIN="1"), capture_output=True, text=True, timeout=110)
+    out = r.stdout.strip().splitlines()
+    assert r.returncode == 0 and out and out[-1].startswith("ok"), r.stdout[-2000:] + r.stderr[-4000:]
+    say(f"[runner] {out[-1]}")
+
+
+def test_runner_prefill_tail_tiles(hip, monkeypatch):
+    """An output product whose last tiles run as K splits that are then added
+    into the residual rows (2100 rows, 8192 columns: 544 tiles, the last 32 of
+    them the last rows'), against the plan without operand tiles, which a
+    workspace limit selects; the last row's logits come from the tail tiles."""
+    from yule_amd.model import LlamaConfig
+    say("[runner] prefill with tail tiles")
+    m = SyntheticModel.generate(LlamaConfig(n_layers=1, dim=8192, n_heads=64, n_kv_heads=8, ff_dim=512, vocab=256,
+                                            max_seq=2112), seed=53, scheme="Q4_K")
+    toks, got = synth.uniform_tokens(54, 2100, 256), []
+    for limit in ("0", "400"):
+        monkeypatch.setenv("YULE_WORKSPACE_LIMIT_MB", limit)
+        run = HipRunner(hip, m)
+        got.append(run.prefill_batched(toks))
+        run.close()
+    # four products in a chain, each side of each within 4e-6 of the exact one
+    # (test_gemm_gpu.py's F32_REL); measured 1.02e-5
+    assert np.linalg.norm(got[0] - got[1]) <= 4 * 2 * 4e-6 * np.linalg.norm(got[1])
+
+
 def test_runner_prefill_determinism_reset_and_limits(hip, tiny):
     say("[runner] prefill determinism / reset / context limit")
     run = HipRunner(hip, tiny)
