@@ -185,6 +185,31 @@ def test_gemm_few_rows_q8_0_small_rows(hip, f32):
             assert rel_error(got[m], ref) <= F32_REL + 2.0 ** -148 * np.sqrt(N) / np.linalg.norm(ref), f"row {m}"
 
 
+@pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
+def test_gemm_few_rows_q8_0_large_partial_sums(hip, f32):
+    """The one-launch kernel where a wave's partial sum passes the f32 range and
+    the result does not: the second 256 columns' weights repeat the first's,
+    their X is the first's times -127/128 (an f32 sum's error then counts 255
+    times)."""
+    N, K, dt = 64, 512, DType.Q8_0
+    say(f"[gemm] few rows Q8_0, large partial sums, {'f32' if f32 else 'bf16'} X")
+    w = synth.gen_quant(dt, 170, N, K, 8.0).reshape(N, 2, -1)
+    w[:, 1] = w[:, 0]
+    x = bf16_to_f32(bf16_bits(synth.gauss(171, (2, 256)))) * np.float32(2.0 ** 123)
+    x = np.concatenate([x, x * np.float32(-127 / 128)], axis=1)
+    if f32:
+        got = run_gemm_f32(hip, dt, w, x, 2, N, K)
+    else:
+        xb = bf16_bits(x)
+        got, x = run_gemm(hip, dt, w, xb, 2, N, K), bf16_to_f32(xb).reshape(2, K)
+    d = w.reshape(N, K // 32, 34)[:, :, :2].copy().view(np.float16).astype(np.float64)
+    wf = (d * w.reshape(N, K // 32, 34)[:, :, 2:].view(np.int8)).reshape(N, K)
+    for m in range(2):
+        part, ref = wf[:, :256] @ x[m, :256].astype(np.float64), wf @ x[m].astype(np.float64)
+        assert np.max(np.abs(part)) > 2.0 ** 128 > 2 * np.max(np.abs(ref))
+        assert rel_error(got[m], ref) <= 255 * F32_REL, f"row {m}"
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 77, 1024), (5, 300, 3072), (16, 64, 2048), (17, 129, 1024),
                                    (32, 200, 3072), (32, 1000, 2048), (8, 4096, 5120), (3, 2000, 14336),
                                    (33, 1000, 2048)])

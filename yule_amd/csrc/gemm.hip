@@ -1598,8 +1598,9 @@ static void *static_workspace(int device) {
 // row's), scaled into f32 accumulators that meet in LDS.  Quants are exact in
 // bf16 and f32 X is the exact sum of three bf16 parts, so only the f32 sums
 // round: a unit of an X row whose magnitudes are all below 2^-63 is raised by
-// 2^96 first, so that no part and no product nears the subnormals.  Bound by the address work of its 8-byte weight reads and of X, which
-// every workgroup reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
+// 2^96 first, so that no part and no product nears the subnormals.  Bound by
+// the address work of its 8-byte weight reads and of X, which every workgroup
+// reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
 // reduction -> this): 256x1024 14.6 -> 4.9, 4096x4096 24.5 -> 16.4 (bf16 X 19.5
 // -> 13.3; one row of f32 X 22.4 -> 12.9).
 //
@@ -1631,7 +1632,11 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
     constexpr uint32_t NW = 16, U = 8;
     constexpr float kDown = 0x1p-12f;   // quants reach 2^7 and a block sums 2^5: its sum stays within the largest |x|
     constexpr float kUp = 0x1p96f;
-    __shared__ __align__(16) float red[NW][256];
+    // the waves' sums times kDown (partial sums may pass the f32 range where
+    // the result does not), and apart from them those of raised units, which
+    // are small; which waves have the latter
+    __shared__ __align__(16) float red[NW][256], red_low[NW][256];
+    __shared__ __align__(16) uint8_t raised[NW];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), n0 = blockIdx.x * 16;
     const uint32_t mr = c < m ? c : m - 1;
@@ -1717,13 +1722,13 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
         }
         return sum;
     };
-    few_f4 acc = {0, 0, 0, 0};
+    few_f4 acc = {0, 0, 0, 0}, low = {0, 0, 0, 0};
     bool again = false;
     // rows whose values in a unit are all below 2^-63 (the two top bits of
     // every exponent are 0) and not all zero: left to the loop after
     auto low_rows = [&](uint32_t top) {
-        const uint64_t low = __ballot(!(top & (F32 ? 0x60000000u : 0x60006000u))), any = __ballot(top != 0);
-        return (uint32_t)(low & (low >> 16) & (low >> 32) & (low >> 48) & (any | any >> 16 | any >> 32 | any >> 48)) & 0xFFFFu;
+        const uint64_t tiny = __ballot(!(top & (F32 ? 0x60000000u : 0x60006000u))), any = __ballot(top != 0);
+        return (uint32_t)(tiny & (tiny >> 16) & (tiny >> 32) & (tiny >> 48) & (any | any >> 16 | any >> 32 | any >> 48)) & 0xFFFFu;
     };
     for (uint32_t u = wave; u < n_cols / 256; u += NW) {
         uint32_t top = 0;
@@ -1731,7 +1736,7 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
         const uint32_t small = low_rows(top);
         again |= small != 0;
 #pragma unroll
-        for (uint32_t r = 0; r < 4; r++) acc[r] += (small >> (4 * g + r)) & 1u ? 0.f : sum[r] * (1.f / kDown);
+        for (uint32_t r = 0; r < 4; r++) acc[r] += (small >> (4 * g + r)) & 1u ? 0.f : sum[r];
     }
     if (again) {
         for (uint32_t u = wave; u < n_cols / 256; u += NW) {
@@ -1744,17 +1749,23 @@ __global__ __launch_bounds__(1024) void gemm_few_q80_kernel(const uint8_t *__res
             if (!small) continue;
             const few_f4 sum = unit(u, std::true_type{}, small, top);
 #pragma unroll
-            for (uint32_t r = 0; r < 4; r++) acc[r] += (small >> (4 * g + r)) & 1u ? sum[r] * (1.f / kDown / kUp) : 0.f;
+            for (uint32_t r = 0; r < 4; r++) low[r] += (small >> (4 * g + r)) & 1u ? sum[r] * (1.f / kDown / kUp) : 0.f;
         }
+        *reinterpret_cast<few_f4 *>(&red_low[wave][4 * lane]) = low;
     }
     *reinterpret_cast<few_f4 *>(&red[wave][4 * lane]) = acc;
+    if (lane == 0) raised[wave] = again;
     __syncthreads();
     const uint32_t on = tid & 15u, om = tid >> 4, row = n0 + on;   // weight row and X row of a thread
     if (om >= m || row >= n_rows) return;                          // m is at most 16
-    float sum = 0.f;
+    const uint32_t at = 4 * ((om >> 2) * 16 + on) + (om & 3u);
+    float sum = 0.f, sum_low = 0.f;
 #pragma unroll
-    for (uint32_t i = 0; i < NW; i++) sum += red[i][4 * ((om >> 2) * 16 + on) + (om & 3u)];
-    y[(size_t)om * n_rows + row] = sum;
+    for (uint32_t i = 0; i < NW; i++) sum += red[i][at];
+    const uint4 any = *reinterpret_cast<const uint4 *>(raised);
+    if (any.x | any.y | any.z | any.w)
+        for (uint32_t i = 0; i < NW; i++) sum_low += raised[i] ? red_low[i][at] : 0.f;
+    y[(size_t)om * n_rows + row] = sum * (1.0f / kDown) + sum_low;
 }
 
 static int launch_gemm_few_q80(hipStream_t s, const uint8_t *w, const void *x, bool f32x, float *y, uint32_t m,
