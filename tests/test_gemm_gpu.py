@@ -388,6 +388,20 @@ def test_gemm_operand_tiles(hip):
     say(f"[gemm] {out[-1]}")
 
 
+# Q6_K with bf16 X, 129..511 rows: shapes on either side of the line between
+# 128- and 256-wide tiles (few tiles, 16, 32 to 64, by cost, one round unsplit)
+@pytest.mark.parametrize("M,N,K", [(132, 612, 3328), (490, 1247, 1280), (129, 2048, 2048), (129, 2048, 1792), (200, 4100, 1024),
+                                   (300, 1536, 4096), (129, 2817, 14336), (140, 14336, 1024), (511, 7000, 2048)])
+def test_gemm_q6k_tile_widths(hip, M, N, K):
+    say(f"[gemm] Q6_K bf16 M={M} N={N} K={K}")
+    w = synth.gen_quant(DType.Q6_K, 180, N, K)
+    xb = bf16_bits(synth.gauss(181 + M, (M, K)))
+    y, xf = run_gemm(hip, DType.Q6_K, w, xb, M, N, K), bf16_to_f32(xb).reshape(M, K)
+    for m in (0, 127, 128, M - 1):
+        ref = oracle.qmv_f64(int(DType.Q6_K), w, xf[m], N, K)
+        assert np.max(np.abs(y[m] - ref)) <= tolerance_bar(ref), f"row {m}"
+
+
 # Q6_K: partials of the 256-wide tiles' K splits that do and do not fit the
 # static workspace (then the 128-wide tiles serve the call)
 @pytest.mark.parametrize("M", [130, 384, 511])

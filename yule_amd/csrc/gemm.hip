@@ -1292,12 +1292,38 @@ namespace {
 // each weight tile is multiplied against and measured 5-30% faster once M
 // fills the CUs with wide tiles (M >= 1024; Q6_K, whose dequant is dearer
 // and whose 128-row kernels run one wave per SIMD either way, from 512, and
-// with bf16 X above 128: 4096 x 14336 at M = 129 94.7 -> 78.5 us, 333 161 -> 119, 4096 x
-// 4096 at M = 400 63 -> 57); 128 (four waves) below that.  YULE_GEMM_BN overrides.
-uint32_t gemm_bn(uint32_t m, uint32_t dtype, bool f32x) {
+// with bf16 X above 128 where q6k_wide says so); 128 (four waves) below that.
+// YULE_GEMM_BN overrides.
+//
+// Q6_K with bf16 X, 129..511 rows: a super-block of a wide tile takes about
+// 1.45 times as long as one of a narrow tile, and a megabyte of split-K
+// partials, of which the wide tiles leave up to twice as much, 0.08 times.
+// Where 32 to 64 wide tiles, or 16 with splits of eight super-blocks and more
+// that differ little, fill the chip, they are ahead without that; fewer than
+// 12 never are.
+// 128 -> 256 wide, us: 333 x 4096 x 14336 158 -> 109, 130 x 4096 x 14336 90 -> 76,
+// 400 x 4096 x 4096 61 -> 54, 256 x 2048 x 2048 29.3 -> 25.6, 400 x 14336 x 1024
+// 59 -> 43; kept narrow: 132 x 612 x 3328 23.6 / 25.9, 320 x 512 x 14336 41.3 /
+// 47.8, 320 x 1536 x 4096 34.9 / 38.7, 256 x 14336 x 1024 33.8 / 39.3.
+bool q6k_wide(uint32_t m, uint32_t n, uint32_t k) {
+    const uint32_t cus = (uint32_t)device_cus(), bpr = k / 256, tall = (m + 127) / 128;
+    const uint32_t tiles = tall * ((n + 255) / 256);
+    if (tiles < 12) return false;
+    const uint32_t even = bpr < 16 ? bpr : (bpr + 15) / 16 * 16;   // super-blocks of 16 equal splits
+    if ((tiles == 16 && bpr >= 8 && 5 * bpr >= 4 * even) || (tiles >= 32 && tiles <= 64)) return true;
+    auto cost = [&](uint32_t t, float per_block) {   // in super-blocks of a narrow tile
+        const uint32_t ks = t >= cus ? 1u : cus / t < bpr ? cus / t : bpr;
+        const float blocks = (float)((t * ks + cus - 1) / cus * ((bpr + ks - 1) / ks));
+        return per_block * blocks + (ks > 1 ? 0.08f * 4e-6f * (float)ks * (float)m * (float)n : 0.f);
+    };
+    return cost(tiles, 1.45f) < cost(tall * ((n + 127) / 128), 1.f);
+}
+
+uint32_t gemm_bn(uint32_t m, uint32_t n, uint32_t k, uint32_t dtype, bool f32x) {
     static const int env = env_int("YULE_GEMM_BN", 0);
     if (env == 128 || env == 256) return (uint32_t)env;
-    return m >= 1024 || (dtype == YULE_DTYPE_Q6_K && (m >= 512 || (!f32x && m > 128))) ? 256u : 128u;
+    if (dtype == YULE_DTYPE_Q6_K && !f32x && m > 128 && m < 512) return q6k_wide(m, n, k) ? 256u : 128u;
+    return m >= 1024 || (dtype == YULE_DTYPE_Q6_K && m >= 512) ? 256u : 128u;
 }
 
 // Tile height: 64 rows for M <= 64, and for f32 X up to M = 128 (its two
@@ -1467,7 +1493,7 @@ static GemmWork gemm_work(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t
                           bool narrow = false) {
     GemmWork g;
     g.q4 = dtype == YULE_DTYPE_Q4_K || dtype == YULE_DTYPE_Q5_K;   // min term: X sub-block sums
-    g.bn = gemm_bn(m, dtype, f32x || narrow);
+    g.bn = gemm_bn(m, n_rows, n_cols, dtype, f32x || narrow);
     g.bm = gemm_bm(m, f32x, dtype, g.bn);
     g.skinny = gemm_skinny(m, n_cols, dtype, f32x);
     g.ks = g.skinny ? gemm_skinny_splits(n_rows, n_cols) : gemm_splits(m, n_rows, n_cols, g.bn, g.bm, gemm_wgs_per_cu(dtype, g.bm, g.bn, f32x));
