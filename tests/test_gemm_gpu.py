@@ -402,6 +402,25 @@ def test_gemm_q6k_tile_widths(hip, M, N, K):
         assert np.max(np.abs(y[m] - ref)) <= tolerance_bar(ref), f"row {m}"
 
 
+# Q6_K on either side of the operand tiles' line: bf16 X by tiles, columns of
+# tiles and rows; f32 X below 512 rows by whole tiles and columns of them
+@pytest.mark.parametrize("M,N,K,f32", [(768, 2048, 8192, False), (768, 2305, 8192, False), (1290, 1100, 11520, False),
+                                       (1270, 1100, 11520, False), (257, 2048, 2816, True), (256, 2048, 4096, True),
+                                       (300, 512, 14336, True)])
+def test_gemm_q6k_operand_tile_line(hip, M, N, K, f32):
+    say(f"[gemm] Q6_K {'f32' if f32 else 'bf16'} X M={M} N={N} K={K}")
+    w, x = synth.gen_quant(DType.Q6_K, 190, N, K), synth.gauss(191 + M, (M, K))
+    if f32:
+        y = run_gemm_f32(hip, DType.Q6_K, w, x, M, N, K)
+    else:
+        xb = bf16_bits(x)
+        y, x = run_gemm(hip, DType.Q6_K, w, xb, M, N, K), bf16_to_f32(xb).reshape(M, K)
+    for m in (0, 128, M - 1):
+        ref = oracle.qmv_f64(int(DType.Q6_K), w, np.ascontiguousarray(x[m]), N, K)
+        assert np.max(np.abs(y[m] - ref)) <= tolerance_bar(ref), f"row {m}"
+        assert not f32 or rel_error(y[m], ref) <= F32_REL, f"row {m}"
+
+
 # Q6_K: partials of the 256-wide tiles' K splits that do and do not fit the
 # static workspace (then the 128-wide tiles serve the call)
 @pytest.mark.parametrize("M", [130, 384, 511])

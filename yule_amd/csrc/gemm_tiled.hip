@@ -700,11 +700,26 @@ int run_pass(hipStream_t s, const TiledPlan &p, const TiledPass &a, uint32_t r_l
 //                 1531 x 2560 x 2048 75 -> 76; Q5_K 1000 x 4096 x 4096 145 -> 124
 //   bf16 X  Q6_K  1531 x 4096 x 4096 139 -> 110, 800 x 4096 x 4096 88 -> 79, 1024 x 2048 x 2048 43 -> 46
 //           the others gain at most 6% at 2048 rows and lose below: gemm.hip
+// Q6_K with f32 X of up to 511 rows by whole tiles of 128 rows and from three
+// columns of tiles on: 200 x 2048 x 4096 51 -> 56, 256 x 4096 x 2048 52 -> 55, 300 x
+// 512 x 14080 72 -> 78, 130 x 3000 x 4096 74 -> 57, 400 x 1200 x 4096 64 -> 57.
+// bf16 X (Q6_K): below 1280 rows of X and 84 tiles the product gains nothing,
+// but where the columns of tiles are a multiple of four from eight on (an XCD
+// then keeps to few of them, and to their weights) and k is long: 776 x 2230 x 8192 97 -> 120, 896 x 1500 x 11520 98 ->
+// 102, 1000 x 1024 x 14336 91 -> 96; 776 x 2048 x 11520 121 -> 103, 776 x 3000 x 11520
+// 148 -> 131, 1300 x 1500 x 11520 144 -> 126.
+// Q4_K of few weight rows gains nothing (2000 x 1024 x 14080 226 -> 243, 1290 x
+// 1024 x 14080 168 -> 165), Q5_K does (180 -> 165).
 static bool tiled_wins(uint32_t m, uint32_t n, uint32_t k, uint32_t dtype, bool f32x) {
     const bool sums = dtype == YULE_DTYPE_Q4_K || dtype == YULE_DTYPE_Q5_K, q6 = dtype == YULE_DTYPE_Q6_K;
     const double work = 1e-9 * m * n * k;
-    if (!f32x) return q6 && m >= 768 && work >= 10;
-    return sums ? m >= 700 && work >= 15 : m > 128 && work >= (q6 ? 1.5 : 3.0);
+    if (!f32x) {
+        const uint32_t cols = (n + kTiledBn - 1) / kTiledBn, tiles = (m + kTiledBm - 1) / kTiledBm * cols;
+        return q6 && m >= 768 && work >= 10 &&
+               (tiles >= 84 || (m >= 1280 && tiles >= 44) || (cols >= 8 && cols % 4 == 0 && k >= 8192));
+    }
+    if (q6 && m < 512) return m > 128 && n > 2 * kTiledBn && 1e-9 * ((m + kTiledBm - 1) / kTiledBm * kTiledBm) * n * k >= 2.25;
+    return sums ? m >= 700 && work >= 15 && (n >= 1536 || dtype == YULE_DTYPE_Q5_K) : m > 128 && work >= (q6 ? 1.5 : 3.0);
 }
 
 bool gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t dtype, bool f32x, TiledPlan *p) {
