@@ -1411,16 +1411,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
 // Phase 2: one workgroup per query head; lanes own four dims and a residue
 // class of the chunks (four in flight), summed through LDS.  118 chunks of 32
 // heads x 128: 10.8 us with one thread per dim walking the chunks, 4.9 us so.
+// FEW: one query head per KV head and at most kCombineFew chunks keep the
+// walk, whose code is short: calls at 512 positions 16/16 heads x 64 6.27 us and
+// 6.73 spread, 32/32 x 64 6.37 and 6.83, 16/16 x 128 7.00 and 7.30; at 1300 (21
+// chunks) 7.07, 7.48, 7.94 and 7.26, 7.62, 7.95, at 2000 level.  With more heads
+// the spread form is ahead from 11 chunks on (32/8 x 80, 700 positions: 10.06 and
+// 9.55) and level below.
 // BASE2: the maxima are of base-2 exponents (attn_split_tile_kernel).
-template <bool BASE2>
+constexpr uint32_t kCombineFew = 24;
+template <bool BASE2, bool FEW>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restrict__ part,
                                                            const float2 *__restrict__ ml,
                                                            const uint32_t *__restrict__ ctl, float *__restrict__ out,
                                                            uint32_t n_kv, uint32_t hd, uint32_t seq_host,
                                                            uint32_t max_chunks) {
-    __shared__ float wt[kSplitMaxChunks];
+    __shared__ float wt[FEW ? kCombineFew : kSplitMaxChunks];
     __shared__ float red[16];
-    __shared__ float4 os[256];
+    __shared__ float4 os[FEW ? 1 : 256];
     const uint32_t h = blockIdx.x, tid = threadIdx.x;
     const uint32_t seq = ctl ? ctl[0] + 1 : seq_host;
     const uint32_t C = BASE2 ? split_tile_chunk(seq, n_kv, hd) : split_chunk(seq, n_kv), n_ch = (seq + C - 1) / C;
@@ -1437,6 +1444,20 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restri
     }
     lsum = block_sum(lsum, red);   // its barriers also publish wt[]
     const float inv = 1.0f / lsum;
+    if constexpr (FEW) {
+        const float *p = part + (size_t)h * max_chunks * hd;
+        for (uint32_t d = tid; d < hd; d += 256) {
+            float a0 = 0.f, a1 = 0.f;
+            uint32_t c = 0;
+            for (; c + 1 < n_ch; c += 2) {
+                a0 += wt[c] * p[(size_t)c * hd + d];
+                a1 += wt[c + 1] * p[(size_t)(c + 1) * hd + d];
+            }
+            if (c < n_ch) a0 += wt[c] * p[(size_t)c * hd + d];
+            out[(size_t)h * hd + d] = (a0 + a1) * inv;
+        }
+        return;
+    }
     const uint32_t nd4 = hd / 4, ng = 256 / nd4, d4 = tid % nd4, gi = tid / nd4;
     const float4 *ph = reinterpret_cast<const float4 *>(part + (size_t)h * max_chunks * hd) + d4;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1949,12 +1970,13 @@ int launch_attn_split(hipStream_t s, const float *q, const float *k, const float
 #undef YULE_SPLIT_ARGS
     int rc = check_launch("attn_split");
     if (rc) return rc;
-    if (tile)
-        hipLaunchKernelGGL(attn_combine_kernel<true>, dim3(n_heads), dim3(256), 0, s, part, ml, ctl, out, n_kv, hd,
-                           seq_host, mc);
-    else
-        hipLaunchKernelGGL(attn_combine_kernel<false>, dim3(n_heads), dim3(256), 0, s, part, ml, ctl, out, n_kv, hd,
-                           seq_host, mc);
+#define YULE_COMBINE(BASE2, FEW)                                                                                     \
+    hipLaunchKernelGGL((attn_combine_kernel<BASE2, FEW>), dim3(n_heads), dim3(256), 0, s, part, ml, ctl, out, n_kv, hd, \
+                       seq_host, mc)
+    if (tile) YULE_COMBINE(true, false);
+    else if (group == 1 && grid.y <= kCombineFew) YULE_COMBINE(false, true);
+    else YULE_COMBINE(false, false);
+#undef YULE_COMBINE
     return check_launch("attn_combine");
 }
 
