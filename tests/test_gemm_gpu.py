@@ -120,10 +120,9 @@ def test_gemm_wide_tiles(hip, dt, M, N, K):
                                    (17, 200, 4096)])
 def test_gemm_few_rows_q8_0(hip, M, N, K):
     """Q8_0, M <= 16: the one-launch kernel (one unit for one wave, nine units
-    over 16 waves, a ragged last tile), bf16 and f32 X, every row vs the
+    and 33 over 16 waves, a ragged last tile), bf16 and f32 X, every row vs the
     oracle; f32 X spread over 60 powers of two and a row near the top of the
-    range, whose outputs are finite; M = 17 and 8448 columns are the tile
-    kernel's."""
+    range, whose outputs are finite; M = 17 is the tile kernel's."""
     dt = DType.Q8_0
     say(f"[gemm] few rows Q8_0 M={M} N={N} K={K}")
     w = synth.gen_quant(dt, 130 + M, N, K)
@@ -141,13 +140,15 @@ def test_gemm_few_rows_q8_0(hip, M, N, K):
             assert N < 30 or rel_error(got[m], ref) <= F32_REL, f"row {m}"   # (bf16 X is exact here)
 
 
-@pytest.mark.parametrize("N,K", [(40, 5632), (4096, 5632), (4097, 5632), (4097, 2816), (8193, 1792), (16384, 1280), (16385, 256),
-                                 (100, 5888)])
+@pytest.mark.parametrize("M,N,K", [(3, 40, 5632), (3, 4096, 12544), (3, 4097, 5632), (3, 4097, 5888), (3, 8193, 3584),
+                                   (3, 8193, 3840), (8, 16384, 2816), (3, 16385, 256), (8, 100, 12544), (9, 100, 9216),
+                                   (3, 100, 12800), (9, 100, 8960), (9, 4097, 4608), (3, 100, 6144)])
 @pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
-def test_gemm_few_rows_q8_0_line(hip, N, K, f32):
+def test_gemm_few_rows_q8_0_line(hip, M, N, K, f32):
     """Either side of the line between the one-launch kernel and the tiles (one,
-    two, three, four and five rounds of workgroups; 22 units over 16 waves)."""
-    dt, M = DType.Q8_0, 3
+    two, three, four and five rounds of workgroups; up to 49 units over 16
+    waves; more than eight rows; a width of whole 2048s)."""
+    dt = DType.Q8_0
     say(f"[gemm] few rows Q8_0 {N}x{K} {'f32' if f32 else 'bf16'} X")
     w, x = synth.gen_quant(dt, 160, N, K), synth.gauss(161 + K, (M, K))
     if f32:
