@@ -211,11 +211,11 @@ def test_gqa_decode_attn_chunk_lengths(hip, hd, nh, nkv, seq):
     run_gqa_case(hip, hd, nh, nkv, seq)
 
 
-@pytest.mark.parametrize("hd,nh,nkv,seq", [(64, 32, 32, 513), (64, 32, 32, 3840), (64, 32, 32, 3841), (128, 8, 8, 16129),
+@pytest.mark.parametrize("hd,nh,nkv,seq", [(64, 32, 32, 513), (64, 32, 32, 3327), (64, 32, 32, 3328), (128, 8, 8, 15359), (128, 8, 8, 16129),
                                           (64, 16, 16, 1536), (64, 16, 16, 1537), (80, 4, 4, 1536), (256, 2, 2, 1537)])
 def test_gqa_decode_attn_one_query_head(hip, hd, nh, nkv, seq):
-    """One query head per KV head: the vector kernel up to the length at which
-    its chunks would be 256 long, the tile kernel from there on; 24 and 25
+    """One query head per KV head: the vector kernel up to a length that goes by
+    the heads, the tile kernel from there on; 24 and 25
     chunks, either side of the end of the combine's walk."""
     say(f"[ops] one query head per KV head, hd={hd} heads={nh}/{nkv} seq={seq}")
     run_gqa_case(hip, hd, nh, nkv, seq)

@@ -1927,15 +1927,18 @@ size_t split_scratch_bytes(uint32_t n_heads, uint32_t hd, uint32_t seq_cap) {
 
 // The tile kernel or the vector one (attn_split_kernel).  With one query head
 // per KV head fifteen of a tile's sixteen columns repeat it, and the vector
-// kernel is ahead until its chunks are 256 long; vector / tile, us (both with
-// the combine): 16 heads x 128: 1615 positions 9.1 / 10.2, 4500 17.5 / 19.6,
-// 11000 70.7 / 32.9; 32 x 64: 1615 9.0 / 10.2, 3300 15.1 / 15.5, 4500 22.6 /
-// 20.0; 8 x 128: 3300 8.9 / 10.3, 11000 21.6 / 21.5.  With two and more the
-// tile kernel is level (16/8 x 128: 1000 9.7 / 9.1, 3300 10.6 / 11.2) to far
-// ahead (12/2 x 128, 3300: 12.4 / 8.8).  A decode step's launch serves every
-// position up to seq_cap and goes by that.
+// kernel is ahead until the chip is well filled; vector / tile, us (both with
+// the combine): 16 heads x 128: 1615 positions 9.1 / 10.2, 4364 17.5 / 19.7,
+// 6348 23.1 / 24.7, 7142 27.0 / 25.2, 11000 70.7 / 32.9; 32 x 128: 2182 17.3 /
+// 20.0, 3571 27.3 / 25.0; 32 x 64: 1190 7.6 / 8.6, 1984 and more level; 8 x 128:
+// 6348 14.8 / 16.2, 14284 25.5 / 26.6, 15713 30.5 / 27.2; 4 x 128: 28569 25.9 /
+// 27.6, 31426 29.0 / 27.8.  With two and more the tile kernel is level (16/8 x
+// 128: 1000 9.7 / 9.1, 3300 10.6 / 11.2) to far ahead (12/2 x 128, 3300: 12.4 /
+// 8.8).  A decode step's launch serves every position up to seq_cap and goes
+// by that.
 static bool split_tile_ok(uint32_t n_heads, uint32_t n_kv, uint32_t hd, uint32_t seq_cap) {
-    return (hd == 64 || hd == 128) && (n_heads > n_kv || split_chunk(seq_cap, n_kv) == 256);
+    return (hd == 64 || hd == 128) &&
+           (n_heads > n_kv || (uint64_t)n_kv * seq_cap >= (n_kv >= 16 ? 104u : 120u) * 1024u);
 }
 
 int launch_attn_split(hipStream_t s, const float *q, const float *k, const float *v, float *kc, float *vc,
