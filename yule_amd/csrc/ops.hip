@@ -1099,8 +1099,8 @@ __global__ __launch_bounds__(NT) void attn_step_kernel(const float *__restrict__
 // the chunk maximum m_c, the sum l_c = sum_t exp(s_t - m_c) and the
 // unnormalised output o_c = sum_t exp(s_t - m_c) V_t; phase 2 combines the
 // chunks: out = sum_c exp(m_c - M) o_c / sum_c exp(m_c - M) l_c.
-// The chunk length is a function of the sequence length and KV heads alone,
-// evaluated on the device in decode steps, so a captured graph sized for
+// The chunk length is a function of the sequence length, the KV heads and the
+// head size alone, evaluated on the device in decode steps, so a captured graph sized for
 // max_seq serves every position; workgroups past the last chunk exit.
 constexpr uint32_t kSplitMaxGroup = 8;      // query heads per KV head
 constexpr uint32_t kSplitMinChunk = 64;
@@ -1875,9 +1875,10 @@ int launch_attn_chunks(hipStream_t s, const float *q, const float *kc, const flo
     const uint32_t C = attn_chunk_len(hd);
     if (!C || !n_kv || n_heads % n_kv) return set_error(YULE_ERR_UNSUPPORTED, "chunked attention: head size");
     // One workgroup per head for 64 dims (a launch serves every position below
-    // max_rows): 100 positions 4.3 us against 6.2 for the chunks, 256 5.2
-    // against 6.2, 500 6.4 against 6.1.  With 128 dims the chunks win from
-    // about 250 positions on (128: 5.5 against 6.0, 500: 9.3 against 6.6).
+    // max_rows): TinyLlama, 16 steps after a prompt, ms with the chunks ->
+    // so: 2 tokens 11.10 -> 10.83, 100 12.67 -> 11.65, 480 17.35 -> 15.35.
+    // With 128 dims the chunks win from about 250 positions on (a launch at
+    // 128: 6.0 us and 5.5, at 500 6.6 and 9.3).
     if (hd == 64 && head_attn_ok(hd, max_rows))
         return launch_attn_head(s, q, nullptr, nullptr, const_cast<float *>(kc), const_cast<float *>(vc), nullptr,
                                 nullptr, ctl, out, n_heads, n_kv, hd, seq_host, max_rows);
@@ -1910,7 +1911,8 @@ bool split_attn_supported(uint32_t n_heads, uint32_t n_kv, uint32_t hd) {
 
 // Sequence length from which attention runs split-KV (environment
 // YULE_ATTN_SPLIT_MIN, default 512); shorter sequences run one workgroup
-// per query head (attn_step_kernel).
+// per query head (attn_head_kernel; head sizes other than 64 and 128
+// attn_step_kernel) or, in the runner at head size 128, the chunked kernel.
 uint32_t attn_split_min_seq() {
     const char *e = getenv("YULE_ATTN_SPLIT_MIN");
     const long v = e ? strtol(e, nullptr, 10) : 0;

@@ -95,6 +95,11 @@ int launch_rope_rows(hipStream_t s, float *q, const float *k, const float *v, fl
 // imbalance of the units), and two units per wave sharing the operand
 // registers (132 us: the cache reads are not the bound, the registers cost
 // waves).  One workgroup per row with vector FMAs took 653 us.
+// A key past a query's position has weight 0 there, but its V row is still
+// multiplied: an infinite or NaN V row makes the up to 15 rows before it in
+// its tile NaN too, besides those from it on.  Nothing that can be read sees
+// the difference: only the last row's logits leave the pass, and that row, as
+// every later position, has the non-finite V row among its own keys.
 template <uint32_t HD, uint32_t NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(HD <= 128 ? 2 : 1))) void attn_prefill_kernel(
     const float *__restrict__ q, const float *__restrict__ kc, const float *__restrict__ vc, float *__restrict__ out,
