@@ -421,16 +421,18 @@ def test_runner_prefill_batched_operand_tiles(hip):
     say(f"[runner] {out[-1]}")
 
 
-def test_runner_prefill_tail_tiles(hip, monkeypatch):
+@pytest.mark.parametrize("rows,ff", [(2100, 512), (704, 8704)])
+def test_runner_prefill_tail_tiles(hip, rows, ff, monkeypatch):
     """An output product whose last tiles run as K splits that are then added
     into the residual rows (2100 rows, 8192 columns: 544 tiles, the last 32 of
-    them the last rows'), against the plan without operand tiles, which a
-    workspace limit selects; the last row's logits come from the tail tiles."""
+    them the last rows'), and gate and up stacked over two passes of 16384 and
+    1024 rows, up's rows on both sides of the cut, against the plan without
+    operand tiles, which a workspace limit selects."""
     from yule_amd.model import LlamaConfig
-    say("[runner] prefill with tail tiles")
-    m = SyntheticModel.generate(LlamaConfig(n_layers=1, dim=8192, n_heads=64, n_kv_heads=8, ff_dim=512, vocab=256,
+    say(f"[runner] prefill of {rows} rows with tail tiles or two passes")
+    m = SyntheticModel.generate(LlamaConfig(n_layers=1, dim=8192, n_heads=64, n_kv_heads=8, ff_dim=ff, vocab=256,
                                             max_seq=2112), seed=53, scheme="Q4_K")
-    toks, got = synth.uniform_tokens(54, 2100, 256), []
+    toks, got = synth.uniform_tokens(54, rows, 256), []
     for limit in ("0", "400"):
         monkeypatch.setenv("YULE_WORKSPACE_LIMIT_MB", limit)
         run = HipRunner(hip, m)

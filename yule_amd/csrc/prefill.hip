@@ -82,9 +82,10 @@ int launch_rope_rows(hipStream_t s, float *q, const float *k, const float *v, fl
 // a wave owns a unit of 16 query rows of one head and walks the keys in
 // sub-tiles of 16 with an online softmax (attn_tile.h).
 //
-// Bound by the f32 matrix rate for long prompts: 1531 rows of 32 heads of 64
-// dims need 9.8 GFLOP of it, 71 us at the ~137 TFLOP/s that this instruction
-// sustains here; measured 112 us.
+// Half bound by the f32 matrix rate for long prompts: 1531 rows of 32 heads of
+// 64 dims need 9.8 GFLOP of it, 62 us at the nominal 157 TFLOP/s; in a prompt
+// pass the launch takes 138 us (127 at best) with the matrix units 47% busy, the
+// softmax between two products in series with them.
 //
 // A workgroup of NW waves owns one unit (head, query tile; the last, longest
 // tiles first).  Its waves take the keys' sub-tiles in turn, with operands
