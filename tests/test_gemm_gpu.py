@@ -140,13 +140,13 @@ def test_gemm_few_rows_q8_0(hip, M, N, K):
             assert N < 30 or rel_error(got[m], ref) <= F32_REL, f"row {m}"   # (bf16 X is exact here)
 
 
-@pytest.mark.parametrize("M,N,K", [(3, 40, 5632), (3, 4096, 12544), (3, 4097, 5632), (3, 4097, 5888), (3, 8193, 3584),
-                                   (3, 8193, 3840), (8, 16384, 2816), (3, 16385, 256), (8, 100, 12544), (9, 100, 9216),
-                                   (3, 100, 12800), (9, 100, 8960), (9, 4097, 4608), (3, 100, 6144)])
+@pytest.mark.parametrize("M,N,K", [(3, 40, 5632), (3, 4096, 14080), (3, 4097, 5632), (3, 4097, 5888), (3, 8193, 3584),
+                                   (3, 8193, 3840), (8, 16384, 2816), (3, 16385, 256), (8, 100, 14080), (9, 100, 12032), (9, 100, 12544),
+                                   (3, 100, 14592), (9, 100, 7168), (9, 100, 9216), (9, 4097, 4608), (3, 100, 6144)])
 @pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
 def test_gemm_few_rows_q8_0_line(hip, M, N, K, f32):
     """Either side of the line between the one-launch kernel and the tiles (one,
-    two, three, four and five rounds of workgroups; up to 49 units over 16
+    two, three, four and five rounds of workgroups; up to 55 units over 16
     waves; more than eight rows; a width of whole 2048s)."""
     dt = DType.Q8_0
     say(f"[gemm] few rows Q8_0 {N}x{K} {'f32' if f32 else 'bf16'} X")

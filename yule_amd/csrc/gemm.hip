@@ -1642,21 +1642,24 @@ static void *static_workspace(int device) {
 //               5632 x 4096   f32 29.2 -> 25.2, 30.7 -> 35.5   bf16 19.9 -> 21.9, 21.7 -> 27.1
 //   four        16384 x 1280  f32 23.6 -> 18.8, 25.6 -> 24.2   bf16 16.5 -> 13.1, 19.3 -> 15.4
 //   eight       32768 x 512   f32 18.1 -> 22.4, 19.1 -> 27.6   bf16 12.3 -> 16.1, 13.4 -> 18.6
-// Rows of X some 2048 columns apart meet the same memory channels, and such
-// widths lose by it from 6144 on; others gain up to about 12000 columns (or
-// columns times rounds), with more than eight rows of X up to about 9000.
+// Rows of X some 2048 columns apart meet the same memory channels (many rows some
+// 1024 apart too), and such widths lose by it from 6144 on; others
+// gain up to about 14000 columns (or 11000, columns times rounds), with more
+// than eight rows of X up to about 12000 (9000).
 // Tiles / this, 2 and 16 rows of X:
 //   one round   2048 x 7168   f32 1.3 1.12   bf16 1.4 1.18     1000 x 10496  f32 1.2 1.03   bf16 1.2 1.08
-//               512 x 9216    f32 1.17 0.90  bf16 1.14 1.02    802 x 11520   f32 1.2 (1094 x 12544 bf16 1.15)
+//               512 x 9216    f32 1.17 0.90  bf16 1.14 1.02    1242 x 12800  f32 1.24 (764 x 14080 bf16 1.03)
 //               512 x 8192    f32 1.00 0.80  bf16 0.91 0.86    2048 x 8192   f32 1.18 0.87  bf16 1.09 0.90
 //   two         8192 x 4864   f32 1.3 1.19   bf16 1.20 1.06    6144 x 4864   f32 1.2 1.04   bf16 1.08 0.94
 //   three       12288 x 3328  f32 1.2 1.16   bf16 1.13 0.99    four  16384 x 2816  f32 1.2 1.05  bf16 1.02 0.90
 constexpr uint32_t kFewRows = 16, kFewRounds = 4;
 static bool few_q80_ok(uint32_t m, uint32_t n_rows, uint32_t n_cols, uint32_t dtype, bool f32x) {
     const uint32_t rounds = (n_rows / 16 + (n_rows % 16 != 0) + (uint32_t)device_cus() - 1) / (uint32_t)device_cus();
-    const uint32_t most = n_cols % 2048 == 0 ? 5632
-                          : m <= 8           ? (rounds == 1 ? 12544 : 11264)
-                                             : (f32x && rounds == 1 ? 8960 : 9216);
+    const uint32_t most = n_cols % 2048 == 0 ? (m <= 8 ? 6144 : 5632)
+                          : m <= 8           ? (rounds == 1 ? 14080 : 11264)
+                          : rounds > 1       ? 9216
+                          : n_cols % 1024    ? 12032
+                                             : (f32x ? 7168 : 9216);
     return dtype == YULE_DTYPE_Q8_0 && m <= kFewRows && rounds <= kFewRounds && (uint64_t)rounds * n_cols <= most;
 }
 
