@@ -164,10 +164,12 @@ def test_gemm_few_rows_q8_0_line(hip, M, N, K, f32):
 def test_gemm_few_rows_q8_0_small_rows(hip, f32):
     """The one-launch kernel on rows far below 1: as exact as ordinary ones down
     to the subnormals (f32 sums of 2304 terms: well under 4e-6), alone, beside
-    ordinary rows, a zero row, and a row whose 256-column units differ."""
+    ordinary rows, a zero row, a row whose 256-column units differ, and weight
+    rows of zeros."""
     N, K, dt = 96, 2304, DType.Q8_0
     say(f"[gemm] few rows Q8_0, small rows, {'f32' if f32 else 'bf16'} X")
     w = synth.gen_quant(dt, 150, N, K)
+    w.reshape(N, -1)[[17, 90]] = 0
     scale = np.float32(2.0) ** np.array([-118, -122, -100, -64, 0, -63, -125, -90, 0], np.float32)
     x = synth.gauss(151, (9, K)) * scale[:, None]
     x[8, 256:] *= np.float32(2.0 ** -120)      # one ordinary unit, eight small ones
@@ -184,6 +186,26 @@ def test_gemm_few_rows_q8_0_small_rows(hip, f32):
         else:
             # results next to the smallest normal f32 carry its spacing, 2^-149
             assert rel_error(got[m], ref) <= F32_REL + 2.0 ** -148 * np.sqrt(N) / np.linalg.norm(ref), f"row {m}"
+
+
+@pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])
+def test_gemm_few_rows_q8_0_non_finite(hip, f32):
+    """The one-launch kernel on infinite and NaN scales and X: rows of X of any
+    magnitude and zero rows give what the sums in f64 give (an infinity may be
+    NaN where its block has quants of both signs or zero)."""
+    N, K, dt = 32, 768, DType.Q8_0
+    say(f"[gemm] few rows Q8_0, non-finite, {'f32' if f32 else 'bf16'} X")
+    w = synth.gen_quant(dt, 175, N, K)
+    d = w.reshape(N, K // 32, 34)[:, :, :2].view(np.float16)
+    d[3, 2], d[5, 9], d[7, 20] = np.inf, np.nan, -np.inf
+    x = bf16_to_f32(bf16_bits(synth.gauss(176, (5, K)))) * np.array([1, 2.0 ** -110, 0, 1, 2.0 ** -110], np.float32)[:, None]
+    x[3, 300], x[4, 300] = np.inf, np.nan
+    got = run_gemm_f32(hip, dt, w, x, 5, N, K) if f32 else run_gemm(hip, dt, w, bf16_bits(x), 5, N, K)
+    bad = np.zeros((5, N), bool)
+    bad[:, [3, 5, 7]] = True
+    bad[3:] = True
+    assert np.array_equal(~np.isfinite(got), bad)
+    assert np.all(np.isnan(got[:, 5])) and np.all(np.isnan(got[2, [3, 7]]))
 
 
 @pytest.mark.parametrize("f32", [False, True], ids=["bf16", "f32"])

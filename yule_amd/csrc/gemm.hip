@@ -1623,9 +1623,10 @@ static void *static_workspace(int device) {
 // (rows = X rows, columns = weight rows, so a lane's block scale is its own
 // row's), scaled into f32 accumulators that meet in LDS.  Quants are exact in
 // bf16 and f32 X is the exact sum of three bf16 parts, so only the f32 sums
-// round: a unit of an X row whose magnitudes are all below 2^-63 is raised by
-// 2^96 first, so that no part and no product nears the subnormals.  Bound by
-// the address work of its 8-byte weight reads and of X, which every workgroup
+// round.  Rows of X below 2^-100, whose parts and products near the subnormals,
+// show in results below 2^-64: then the workgroup looks at X, and rows that lie
+// below 2^-63 are done again raised by 2^96 (looking at X first cost up to 12%:
+// 6 x 3756 x 1280 f32 X 4.8 -> 5.4 us).  Bound by the address work of its 8-byte weight reads and of X, which every workgroup
 // reads anew.  13 rows of f32 X (us; pre-pass, tile kernel and
 // reduction -> this): 256x1024 14.6 -> 4.9, 4096x4096 24.5 -> 16.4 (bf16 X 19.5
 // -> 13.3; one row of f32 X 22.4 -> 12.9).
@@ -1674,22 +1675,31 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
                                                             uint32_t n_cols) {
     constexpr uint32_t NW = 16, U = 8;
     constexpr float kDown = 0x1p-12f;   // quants reach 2^7 and a block sums 2^5: its sum stays within the largest |x|
-    constexpr float kUp = 0x1p96f;
-    // the waves' sums times kDown (partial sums may pass the f32 range where
-    // the result does not), and apart from them those of raised units, which
-    // are small; which waves have the latter
-    __shared__ __align__(16) float red[NW][256], red_low[NW][256];
-    __shared__ __align__(16) uint8_t raised[NW];
+    constexpr float kUp = 0x1p96f, kLow = 0x1p-64f;
+    __shared__ __align__(16) float red[NW][256];
+    __shared__ uint32_t looked, tops[16];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, c = lane & 15u, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), n0 = blockIdx.x * 16;
     const uint32_t mr = c < m ? c : m - 1;
     const uint8_t *wr = w + (size_t)(n0 + c < n_rows ? n0 + c : n_rows - 1) * (n_cols / 32) * 34;
     const float *xf = static_cast<const float *>(xv) + (size_t)mr * n_cols + 8 * g;
     const uint16_t *xh = static_cast<const uint16_t *>(xv) + (size_t)mr * n_cols + 8 * g;
-    // one unit of 256 columns: the sums of the lane's column and rows 4 g + r.
-    // raise (wave-uniform): the rows in the bits of `small` times kUp first.
-    // top: the OR of the lane's X bits
-    auto unit = [&](uint32_t u, auto raise, uint32_t small, uint32_t &top) {
+    // two quants a dword, the upper halves of their floats
+    auto quants = [&](const uint2 &q) {
+        uint32_t wq[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const uint32_t v = (i < 2 ? q.x : q.y) >> (16 * (i & 1u));
+            wq[i] = __builtin_amdgcn_perm(__float_as_uint((float)(int8_t)(v >> 8) * kDown),
+                                          __float_as_uint((float)(int8_t)v * kDown), 0x07060302u);
+        }
+        bf8v bw;
+        __builtin_memcpy(&bw, wq, 16);
+        return bw;
+    };
+    // one unit of 256 columns added to the sums of the lane's column and rows 4
+    // g + r; raise: X times up first (f32 X)
+    auto unit = [&](uint32_t u, few_f4 sum, auto raise, float up) {
         uint2 qs[U];
         uint16_t ds[U];
         float4 xr[F32 ? 2 * U : U];
@@ -1706,17 +1716,11 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
                 xr[b] = *reinterpret_cast<const float4 *>(xh + u * 256 + b * 32);
             }
         }
-        const float up = (small >> c) & 1u ? kUp : 1.f;
-        few_f4 sum = {0, 0, 0, 0};
 #pragma unroll
         for (uint32_t b = 0; b < U; b++) {
             // X as bf16 parts (one, or three that sum to the f32 exactly)
             constexpr uint32_t NP = F32 ? 3 : 1;
             bf8v a[NP];
-            uint32_t xb[F32 ? 8 : 4];
-            __builtin_memcpy(xb, &xr[F32 ? 2 * b : b], sizeof(xb));
-#pragma unroll
-            for (uint32_t i = 0; i < (F32 ? 8 : 4); i++) top |= xb[i];
             if constexpr (F32) {
                 float x[8] = {xr[2 * b].x,     xr[2 * b].y,     xr[2 * b].z,     xr[2 * b].w,
                               xr[2 * b + 1].x, xr[2 * b + 1].y, xr[2 * b + 1].z, xr[2 * b + 1].w};
@@ -1736,23 +1740,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
                     for (uint32_t i = 0; i < 8; i++) x[i] -= __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
                 }
             } else {
-                if constexpr (decltype(raise)::value) {
-#pragma unroll
-                    for (uint32_t i = 0; i < 4; i++)
-                        xb[i] = __builtin_amdgcn_perm(__float_as_uint(__uint_as_float(xb[i] & 0xFFFF0000u) * up),
-                                                      __float_as_uint(__uint_as_float(xb[i] << 16) * up), 0x07060302u);
-                }
-                __builtin_memcpy(&a[0], xb, 16);
+                __builtin_memcpy(&a[0], &xr[b], 16);
             }
-            uint32_t wq[4];
-#pragma unroll
-            for (uint32_t i = 0; i < 4; i++) {   // two quants a dword, the upper halves of their floats
-                const uint32_t v = (i < 2 ? qs[b].x : qs[b].y) >> (16 * (i & 1u));
-                wq[i] = __builtin_amdgcn_perm(__float_as_uint((float)(int8_t)(v >> 8) * kDown),
-                                              __float_as_uint((float)(int8_t)v * kDown), 0x07060302u);
-            }
-            bf8v bw;
-            __builtin_memcpy(&bw, wq, 16);
+            const bf8v bw = quants(qs[b]);
             few_f4 t = {0, 0, 0, 0};
 #pragma unroll
             for (uint32_t part = 0; part < NP; part++)
@@ -1765,50 +1755,73 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
         }
         return sum;
     };
-    few_f4 acc = {0, 0, 0, 0}, low = {0, 0, 0, 0};
-    bool again = false;
-    // rows whose values in a unit are all below 2^-63 (the two top bits of
-    // every exponent are 0) and not all zero: left to the loop after
-    auto low_rows = [&](uint32_t top) {
-        const uint64_t tiny = __ballot(!(top & (F32 ? 0x60000000u : 0x60006000u))), any = __ballot(top != 0);
-        return (uint32_t)(tiny & (tiny >> 16) & (tiny >> 32) & (tiny >> 48) & (any | any >> 16 | any >> 32 | any >> 48)) & 0xFFFFu;
-    };
-    for (uint32_t u = wave; u < n_cols / 256; u += NW) {
-        uint32_t top = 0;
-        const few_f4 sum = unit(u, std::false_type{}, 0u, top);
-        const uint32_t small = low_rows(top);
-        again |= small != 0;
-#pragma unroll
-        for (uint32_t r = 0; r < 4; r++) acc[r] += (small >> (4 * g + r)) & 1u ? 0.f : sum[r];
-    }
-    if (again) {
-        for (uint32_t u = wave; u < n_cols / 256; u += NW) {
-            uint32_t top = 0;
-            for (uint32_t b = 0; b < U; b++)
-                for (uint32_t i = 0; i < (F32 ? 8 : 4); i++)
-                    top |= F32 ? __float_as_uint(xf[u * 256 + b * 32 + i])
-                               : reinterpret_cast<const uint32_t *>(xh + u * 256 + b * 32)[i];
-            const uint32_t small = low_rows(top);
-            if (!small) continue;
-            const few_f4 sum = unit(u, std::true_type{}, small, top);
-#pragma unroll
-            for (uint32_t r = 0; r < 4; r++) low[r] += (small >> (4 * g + r)) & 1u ? sum[r] * (1.f / kDown / kUp) : 0.f;
-        }
-        *reinterpret_cast<few_f4 *>(&red_low[wave][4 * lane]) = low;
+    const few_f4 zero = {0, 0, 0, 0};
+    few_f4 acc = zero;
+    for (uint32_t u = wave; u < n_cols / 256; u += NW) {   // (bf16 X has no registers for sums of its own)
+        if constexpr (F32) acc += unit(u, zero, std::false_type{}, 1.f);
+        else acc = unit(u, acc, std::false_type{}, 1.f);
     }
     *reinterpret_cast<few_f4 *>(&red[wave][4 * lane]) = acc;
-    if (lane == 0) raised[wave] = again;
+    if (tid == 0) looked = 0;
+    if (tid < 16) tops[tid] = 0;
     __syncthreads();
-    const uint32_t on = tid & 15u, om = tid >> 4, row = n0 + on;   // weight row and X row of a thread
-    if (om >= m || row >= n_rows) return;                          // m is at most 16
-    const uint32_t at = 4 * ((om >> 2) * 16 + on) + (om & 3u);
-    float sum = 0.f, sum_low = 0.f;
+    // weight row and X row of a thread (m is at most 16); the waves' sums are
+    // times kDown: one may pass the f32 range where the result does not
+    const uint32_t on = tid & 15u, om = tid >> 4, row = n0 + on;
+    const bool mine = om < m && row < n_rows;
+    auto total = [&]() {
+        float sum = 0.f;
 #pragma unroll
-    for (uint32_t i = 0; i < NW; i++) sum += red[i][at];
-    const uint4 any = *reinterpret_cast<const uint4 *>(raised);
-    if (any.x | any.y | any.z | any.w)
-        for (uint32_t i = 0; i < NW; i++) sum_low += raised[i] ? red_low[i][at] : 0.f;
-    y[(size_t)om * n_rows + row] = sum * (1.0f / kDown) + sum_low;
+        for (uint32_t i = 0; i < NW; i++) sum += red[i][4 * ((om >> 2) * 16 + on) + (om & 3u)];
+        return sum;
+    };
+    const float sum = mine ? total() : 0.f;
+    if (mine) y[(size_t)om * n_rows + row] = sum * (1.f / kDown);
+    // (all sixteen columns of a row: a weight row of zeros is no reason to look)
+    if ((__ballot(fabsf(sum) < kLow * kDown) >> (lane & 48u) & 0xFFFFu) == 0xFFFFu && om < m) looked = 1;
+    __syncthreads();
+    if (!looked) return;
+    uint32_t top = 0;   // the OR of a row's bits: the two top bits of every exponent are 0 below 2^-63
+    for (uint32_t u = wave; u < n_cols / 256; u += NW)
+#pragma unroll 1
+        for (uint32_t b = 0; b < U; b++)
+            for (uint32_t i = 0; i < (F32 ? 8 : 4); i++)
+                top |= F32 ? __float_as_uint(xf[u * 256 + b * 32 + i])
+                           : reinterpret_cast<const uint32_t *>(xh + u * 256 + b * 32)[i];
+    atomicOr(&tops[c], top);
+    __syncthreads();
+    const uint32_t small = (uint32_t)__ballot(tops[c] != 0 && !(tops[c] & (F32 ? 0x60000000u : 0x60006000u))) & 0xFFFFu;
+    if (!small) return;
+    acc = zero;
+    const float up = (small >> c) & 1u ? kUp : 1.f;
+    for (uint32_t u = wave; u < n_cols / 256; u += NW) {
+        if constexpr (F32) {
+            acc += unit(u, zero, std::true_type{}, up);
+        } else {
+#pragma unroll 1
+            for (uint32_t b = 0; b < U; b++) {   // one block in flight: a whole unit spills at 64 registers
+                const uint8_t *blk = wr + (size_t)(u * U + b) * 34;
+                _Float16 d;
+                uint2 q;
+                uint32_t xb[4];
+                __builtin_memcpy(&d, blk, 2);
+                __builtin_memcpy(&q, blk + 2 + 8 * g, 8);
+                __builtin_memcpy(xb, xh + u * 256 + b * 32, 16);
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++)
+                    xb[i] = __builtin_amdgcn_perm(__float_as_uint(__uint_as_float(xb[i] & 0xFFFF0000u) * up),
+                                                  __float_as_uint(__uint_as_float(xb[i] << 16) * up), 0x07060302u);
+                bf8v a;
+                __builtin_memcpy(&a, xb, 16);
+                const few_f4 t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, quants(q), zero, 0, 0, 0);
+#pragma unroll
+                for (uint32_t r = 0; r < 4; r++) acc[r] += (float)d * t[r];
+            }
+        }
+    }
+    *reinterpret_cast<few_f4 *>(&red[wave][4 * lane]) = acc;
+    __syncthreads();
+    if (mine && (small >> om) & 1u) y[(size_t)om * n_rows + row] = total() * (1.f / kDown / kUp);
 }
 
 static int launch_gemm_few_q80(hipStream_t s, const uint8_t *w, const void *x, bool f32x, float *y, uint32_t m,
